@@ -176,6 +176,92 @@ __device__ __forceinline__ StageMap stage_row(const kr_half* __restrict__ rp, in
     return sm;
 }
 
+// ---------------------------------------------------------------------------
+// Whole CDF (or count) rows leave through LDS. A thread holds counts of
+// scattered leaves, 8 consecutive elements per 8-lane group, and a row of
+// int32 starts at any 4-byte address, so stores from that layout write 32-byte
+// pieces and a scan over them in memory reads lanes 200 bytes apart. Instead
+// the counts of up to 32768 elements at a time (4 blocks of the summation, so
+// no leaf is split) go into the stage, which the gathered row has left; every
+// thread scans one run of kSpanRun elements there, and the results are stored
+// with consecutive lanes on consecutive words. Element i of a span sits at
+// word i + 4 (i / 32): the 16-byte reads of 16 neighbouring runs (36 words
+// apart) then hit all banks once.
+// Bound: the row's own VALU phases (about 20 us per row and CU). Measured on
+// MI355X, 300 rows x 50277: 447 us from the leaf layout, 79 us through LDS (256
+// rows, one per CU: 45 us, of which 13 us are the output).
+// ---------------------------------------------------------------------------
+constexpr int kSpan = 32768;
+constexpr int kSpanRun = kSpan / kThreads;
+constexpr int kSpanWords = kSpan + kSpan / 8;
+__device__ __forceinline__ int span_pos(int i) { return i + ((i >> 5) << 2); }
+
+// Scan (SCAN) or leave as they are n counts in `cnt`, add `carry`, and store
+// them at orow[0 .. n). Returns the last inclusive sum. Every thread calls it;
+// the counts were written by the callers' threads before.
+template <bool SCAN>
+__device__ __forceinline__ int span_out(int* cnt, int n, int carry, int32_t* __restrict__ orow,
+                                        int* redi, int tid, int lane, int wave) {
+    static_assert(kSpanRun == 32, "a run is one skew segment");
+    __syncthreads();
+    if constexpr (SCAN) {
+        // two passes over the run in LDS (its sum, then its prefix sums): the
+        // q values still held leave no registers for 32 counts
+        const int i0 = tid * kSpanRun;
+        int4* run = reinterpret_cast<int4*>(cnt + span_pos(i0));
+        auto quad = [&](int q) {                 // words past n hold no count
+            int4 w = run[q];
+            const int i = i0 + 4 * q;
+            w.x = i < n ? w.x : 0;
+            w.y = i + 1 < n ? w.y : 0;
+            w.z = i + 2 < n ? w.z : 0;
+            w.w = i + 3 < n ? w.w : 0;
+            return w;
+        };
+        int local = 0;
+        #pragma unroll 4
+        for (int q = 0; q < kSpanRun / 4; q++) {
+            const int4 w = quad(q);
+            local += (w.x + w.y) + (w.z + w.w);
+        }
+        int incl = local;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(incl, o);
+            if (lane >= o) incl += up;
+        }
+        if (lane == 63) redi[wave] = incl;
+        __syncthreads();
+        int base = carry + incl - local;
+        int all = carry;
+        for (int w = 0; w < kWaves; w++) {
+            if (w < wave) base += redi[w];
+            all += redi[w];
+        }
+        #pragma unroll 4
+        for (int q = 0; q < kSpanRun / 4; q++) {
+            int4 w = quad(q);
+            w.x += base;
+            w.y += w.x;
+            w.z += w.y;
+            w.w += w.z;
+            base = w.w;
+            run[q] = w;
+        }
+        carry = all;
+        __syncthreads();
+    }
+    // eight words per thread read before they are stored
+    for (int i0 = tid; i0 < n; i0 += 8 * kThreads) {
+        int c[8];
+        #pragma unroll
+        for (int u = 0; u < 8; u++) c[u] = cnt[span_pos(min(i0 + u * kThreads, n - 1))];
+        #pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (i0 + u * kThreads < n) orow[i0 + u * kThreads] = c[u];
+    }
+    return carry;
+}
+
 // The summation plan into LDS: all loads issued before the LDS writes.
 __device__ __forceinline__ void copy_plan(const PlanArgs& P, RowShared& sh, int tid) {
     const bool a = tid < P.n_inner, b = tid <= P.n_levels, c = tid < P.n_blocks,
@@ -566,10 +652,6 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
             const float p = div_by(v[it][k], denom, rdenom);
             const int f = scaled_floor<IN>(p, scale);
             ls += f;
-            if constexpr (MODE == M_CDF || MODE == M_COUNTS) {
-                const bool live = k < 16 ? (k < nf) : (j < rm);
-                if (live) orow[slot_index(start[it], len[it], j, k) + 1] = f + 1;
-            }
             any_hit[it] = any_hit[it] || is_hit(it, k, p);
         }
         lsum[it] = ls + nf + (j < rm ? 1 : 0);
@@ -657,10 +739,7 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
         sh.amax = gi;
         sh.deficit = deficit;
         sh.amax_leaf = gL;
-        if constexpr (MODE == M_CDF || MODE == M_COUNTS) {
-            orow[gi + 1] += deficit;
-            orow[0] = 0;
-        }
+        if constexpr (MODE == M_CDF || MODE == M_COUNTS) orow[0] = 0;
         if constexpr (MODE == M_PAIRS) {
             int pre = 0, cs = 0;
             for (int w = 0; w < kWaves; w++) { pre += sh.redi3[w]; cs += sh.redL[w]; }
@@ -670,27 +749,41 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
         }
         if constexpr (MODE == M_DECODE) sh.leaf_count[gL] += deficit;
     }
-    if constexpr (MODE == M_PAIRS || MODE == M_COUNTS) return;
+    if constexpr (MODE == M_PAIRS) return;
 
-    if constexpr (MODE == M_CDF) {
-        // Inclusive scan of counts over contiguous per-thread segments.
+    if constexpr (MODE == M_CDF || MODE == M_COUNTS) {
         __syncthreads();
-        const int seg = (V + kThreads - 1) / kThreads;
-        const int i0 = min(V, tid * seg), i1 = min(V, i0 + seg);
-        int local = 0;
-        for (int i = i0; i < i1; i++) local += orow[i + 1];
-        int incl = local;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int up = __shfl_up(incl, o);
-            if (lane >= o) incl += up;
-        }
-        if (lane == 63) sh.redi[wave] = incl;
-        __syncthreads();
-        int base = incl - local;
-        for (int w = 0; w < wave; w++) base += sh.redi[w];
-        for (int i = i0; i < i1; i++) {
-            base += orow[i + 1];
-            orow[i + 1] = base;
+        const int gi = sh.amax, deficit = sh.deficit;
+        int* cnt = reinterpret_cast<int*>(stage);
+        int carry = 0;
+        // the q values become counts (same operations, same bits as above)
+        #pragma unroll
+        for (int it = 0; it < kMaxIt; it++)
+            if (act[it]) {
+                #pragma unroll
+                for (int k = 0; k < 17; k++)
+                    v[it][k] = __builtin_bit_cast(
+                        float, scaled_floor<IN>(div_by(v[it][k], denom, rdenom), scale) + 1);
+            }
+        for (int s0 = 0; s0 < V; s0 += kSpan) {
+            if (s0 > 0) __syncthreads();   // the previous span has been stored
+            #pragma unroll
+            for (int it = 0; it < kMaxIt; it++) {
+                if (!act[it] || len[it] == 0 || start[it] < s0 || start[it] >= s0 + kSpan) continue;
+                const int nf = leaf_full(len[it]), rm = leaf_rem(len[it]);
+                #pragma unroll
+                for (int k = 0; k < 17; k++) {
+                    const bool live = k < 16 ? (k < nf) : (j < rm);
+                    const int idx = slot_index(start[it], len[it], j, k) - s0;
+                    if (live) cnt[span_pos(idx)] = __builtin_bit_cast(int, v[it][k]);
+                }
+            }
+            if (gi >= s0 && gi < s0 + kSpan) {   // uniform: the maximum takes the deficit
+                __syncthreads();
+                if (tid == 0) cnt[span_pos(gi - s0)] += deficit;
+            }
+            carry = span_out<MODE == M_CDF>(cnt, min(kSpan, V - s0), carry, orow + s0 + 1, sh.redi,
+                                            tid, lane, wave);
         }
         return;
     }
@@ -804,13 +897,21 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
     }
 }
 
+// Halves of stage a kernel needs: the staged fp16 row, or the counts of a span.
+template <int IN, int MODE>
+constexpr int kStageUsed = MODE == M_CDF || MODE == M_COUNTS ? 2 * kSpanWords
+                           : IN == IN_LOGITS_F16            ? kStageMax
+                                                            : 8;
+static_assert(2 * kSpanWords >= kStageMax && 4 * kSpanWords + sizeof(RowShared) <= 160 * 1024,
+              "the stage of a full-row kernel holds a row or a span of counts, in a CU's LDS");
+
 template <int IN, int MODE>
 __global__ void __launch_bounds__(kThreads)
 row_cdf_kernel(const void* __restrict__ input, long long ld, int n_rows, PlanArgs P, int prec,
                void* __restrict__ out, long long out_ld, const int32_t* __restrict__ symbols,
                DecodeArgs D, int async_stage) {
     __shared__ RowShared sh;
-    __shared__ __attribute__((aligned(16))) kr_half stage[IN == IN_LOGITS_F16 ? kStageMax : 8];
+    __shared__ __attribute__((aligned(16))) kr_half stage[kStageUsed<IN, MODE>];
     const int tid = threadIdx.x;
     if constexpr (MODE != M_DECODE) copy_plan(P, sh, tid);   // decode copies it after its first loads
     const unsigned stage_lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)stage;

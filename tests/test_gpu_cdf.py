@@ -148,3 +148,21 @@ def test_fused_decode_matches_oracle():
         n = int(ntok[b])
         np.testing.assert_array_equal(got[b, :n], syms[b, :n])
     assert cnt.cpu().tolist() == [N, N, N - 5, N]
+
+
+@pytest.mark.parametrize("V", [1, 127, 128, 8193, 32767, 32768, 32769, 32905, 65032, 65536])
+def test_full_rows_at_span_edges(V):
+    """Whole CDF and count rows leave in spans of 32768 counts, each thread
+    scanning 32: vocabularies around one span, with the maximum (which takes
+    the deficit) in the first, the last and a middle element. Integers: exact."""
+    lg = _logits(3, V, V, 3.0)
+    for r, i in enumerate((0, V - 1, V // 2)):
+        lg[r, i] = 14.0
+    d = torch.from_numpy(lg).to(DEV)
+    ref = osm.logits_to_cdf(lg)
+    np.testing.assert_array_equal(ops.softmax_cdf(d).cpu().numpy().view(np.uint32), ref)
+    counts = ops.det_softmax_cdf(d, 1 << 24).cpu().numpy()
+    assert (counts[:, 0] == 0).all()
+    np.testing.assert_array_equal(counts[:, 1:], np.diff(ref.astype(np.int64), axis=1))
+    q = osm.softmax_probs(lg)
+    np.testing.assert_array_equal(krunch_ac.probs_to_cdf(q), ref)
