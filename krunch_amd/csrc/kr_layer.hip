@@ -23,6 +23,7 @@
 #include "kr_model.h"
 #include "kr_rowops.h"
 #include "kr_wave.h"
+#include "kr_wkv.h"
 
 namespace {
 
@@ -143,87 +144,6 @@ ln_mix_kernel(LnMixArgs a) {
             store_row<G>(a.state + (size_t)b * C, lane, cur);
         }
     }
-}
-
-// ---------------------------------------------------------------------------
-// WKV recurrence (wkv_kernel.cu:52-73 semantics), one lane per (stream,
-// channel), sequential over T; fused with the receptance product:
-// ry = fp16(r * fp16(y)), written row-major or fragment-packed (ry_frag) for
-// the output projection. State aa, bb, pp is read once and written once.
-// ---------------------------------------------------------------------------
-constexpr int kWkvChunk = 16;
-
-struct WkvState {
-    float a, b, p;
-};
-
-// One token of the recurrence; returns ry.
-// DET: exps by kr_kexp and an IEEE division (the w8a8 codec, which the oracle
-// restates bit for bit; every exp argument here is <= 0). Otherwise (the fp16
-// codec) the hardware exp and the quotient as numerator times the hardware
-// reciprocal (~1 ulp; y is rounded to fp16 next): the packed and stepped
-// paths both run this function, so their bits agree.
-template <bool DET>
-__device__ __forceinline__ kr_half wkv_token(WkvState& st, float w, float u, float kk, float vv,
-                                             float rr) {
-    const float ww = u + kk;
-    const float p1 = fmaxf(st.p, ww);
-    const float e1 = kr_exp_t<DET>(st.p - p1), e2 = kr_exp_t<DET>(ww - p1);
-    const float num = e1 * st.a + e2 * vv, den = e1 * st.b + e2;   // den >= min(1, bb) > 0
-    float y;
-    if constexpr (DET) y = num / den;
-    else y = num * __builtin_amdgcn_rcpf(den);
-    const kr_half ry = kr_f16(rr * (float)kr_f16(y));
-    const float ww2 = w + st.p;
-    const float p2 = fmaxf(ww2, kk);
-    const float f1 = kr_exp_t<DET>(ww2 - p2), f2 = kr_exp_t<DET>(kk - p2);
-    st.a = f1 * st.a + f2 * vv;
-    st.b = f1 * st.b + f2;
-    st.p = p2;
-    return ry;
-}
-
-template <bool DET>
-__global__ void __launch_bounds__(256) wkv_kernel(const float* __restrict__ k,
-                                                  const float* __restrict__ v,
-                                                  const kr_half* __restrict__ r,
-                                                  const float* __restrict__ decay,
-                                                  const float* __restrict__ first,
-                                                  float* __restrict__ aa, float* __restrict__ bb,
-                                                  float* __restrict__ pp, kr_half* __restrict__ ry,
-                                                  int B, int T, int C, int ry_frag) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    const int b = blockIdx.y;
-    if (c >= C || b >= B) return;
-    const size_t s = (size_t)b * C + c;
-    const size_t base = (size_t)b * T * C + c;
-    const float w = decay[c], u = first[c];
-    WkvState st{aa[s], bb[s], pp[s]};
-    auto ry_at = [&](int t) -> size_t {
-        return ry_frag ? kr_frag_index((long long)b * T + t, c, C) : base + (size_t)t * C;
-    };
-    // A chunk's loads are unconditional (tokens past T re-read token T-1) and
-    // r stays fp16 until its token is computed, so all 3 x kWkvChunk loads are
-    // in flight at once. A load under `t < T` with its conversion beside it
-    // makes the compiler wait for each token's loads in turn (one memory
-    // latency per token).
-    for (int t0 = 0; t0 < T; t0 += kWkvChunk) {
-        float kk[kWkvChunk], vv[kWkvChunk];
-        kr_half rh[kWkvChunk];
-        #pragma unroll
-        for (int q = 0; q < kWkvChunk; q++) {
-            const size_t i = base + (size_t)min(t0 + q, T - 1) * C;
-            kk[q] = k[i];
-            vv[q] = v[i];
-            rh[q] = r[i];
-        }
-        #pragma unroll
-        for (int q = 0; q < kWkvChunk; q++)
-            if (t0 + q < T) ry[ry_at(t0 + q)] = wkv_token<DET>(st, w, u, kk[q], vv[q], (float)rh[q]);
-    }
-    aa[s] = st.a;
-    bb[s] = st.b;
-    pp[s] = st.p;
 }
 
 // ---------------------------------------------------------------------------
@@ -589,6 +509,12 @@ Work carve(void* ws, long long M, int C, int F) {
     return w;
 }
 
+kr_wkv_args wkv_args(const kr_layer_weights& L, const kr_layer_state& st, const Work& w, int B,
+                     int T, int C, bool ry_frag) {
+    return kr_wkv_args{w.k, w.v, w.r, L.decay, L.first, st.aa, st.bb, st.pp, w.ry, B, T, C,
+                       ry_frag ? 1 : 0};
+}
+
 int rows_per_run(int T) { return T >= 64 ? 16 : (T >= 8 ? 4 : 1); }
 
 kr_gemm_args gemm_args(const kr_half* A, int M, int K, const void* Wt, int N, void* out,
@@ -823,10 +749,7 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
             KR_TRY(kr_gemm_launch_multi(jobs, eps, 3, s));
         }
         KR_TRY(ph.mark(2));
-        dim3 grid((C + 255) / 256, B);
-        wkv_kernel<true><<<grid, 256, 0, s>>>(w.k, w.v, w.r, L.decay, L.first, st.aa, st.bb, st.pp,
-                                        w.ry, B, T, C, fr ? 1 : 0);
-        KR_LAUNCHED();
+        KR_TRY(kr_wkv_launch(wkv_args(L, st, w, B, T, C, fr), true, s));
     }
     KR_TRY(ph.mark(3));
     if (fr) {
@@ -970,12 +893,7 @@ int layer_forward(const kr_layer_weights& L, int C, int F, kr_half* x, int B, in
         KR_TRY(kr_gemm_launch_multi(jobs, eps, 3, s));
     }
     KR_TRY(ph.mark(2));
-    {
-        dim3 grid((C + 255) / 256, B);
-        wkv_kernel<false><<<grid, 256, 0, s>>>(w.k, w.v, w.r, L.decay, L.first, st.aa, st.bb, st.pp,
-                                        w.ry, B, T, C, fr ? 1 : 0);
-        KR_LAUNCHED();
-    }
+    KR_TRY(kr_wkv_launch(wkv_args(L, st, w, B, T, C, fr), false, s));
     KR_TRY(ph.mark(3));
     KR_TRY(kr_gemm_launch(gemm_args(w.ry, M, C, L.Ot, C, x, x, nullptr, L.Of, fr), KR_EP_RESID, s));
     KR_TRY(ph.mark(4));
@@ -1453,20 +1371,6 @@ int kr_step_timing_read(double* launch_us, double* span_us, int n, int* n_read) 
     }
     if (n_read) *n_read = k;
     g_step.n = 0;
-    return KR_OK;
-}
-
-int kr_wkv(int B, int T, int C, const float* decay, const float* first, const float* k,
-           const float* v, const uint16_t* r, float* aa, float* bb, float* pp, uint16_t* ry,
-           void* stream) {
-    KR_REQUIRE(decay && first && k && v && r && aa && bb && pp && ry, "kr_wkv: null pointer");
-    KR_REQUIRE(B >= 1 && T >= 0 && C >= 1, "kr_wkv: bad shape");
-    if (T == 0) return KR_OK;
-    dim3 grid((C + 255) / 256, B);
-    wkv_kernel<false><<<grid, 256, 0, kr_stream(stream)>>>(k, v, reinterpret_cast<const kr_half*>(r),
-                                                    decay, first, aa, bb, pp,
-                                                    reinterpret_cast<kr_half*>(ry), B, T, C, 0);
-    KR_LAUNCHED();
     return KR_OK;
 }
 
