@@ -515,7 +515,20 @@ kr_wkv_args wkv_args(const kr_layer_weights& L, const kr_layer_state& st, const 
                        ry_frag ? 1 : 0};
 }
 
-int rows_per_run(int T) { return T >= 64 ? 16 : (T >= 8 ? 4 : 1); }
+// Rows a wave of LN-mix takes in turn. A run shares the loads of its
+// coefficients and of each row's predecessor, but its rows wait on memory one
+// after the other, so short runs as long as the launch has fewer than ~2048
+// waves (two per SIMD). Measured on MI355X, one layer over one stream of M
+// rows, us at 1 / 2 / 4 / 16 rows per run: M = 1024 146 / 148 / 152 / 177,
+// 2048 194 / 194 / 199 / 223, 4096 325 / 324 / 326 / 351, 8192 500 / 495 /
+// 493 / 513, 20480 1212 / 1192 / 1195 / 1213, 65536 4159 / 4105 / 4116 / 4110
+// (8: 4094). Runs never cross streams: T caps them, as before (T < 8 one row,
+// T < 64 four).
+int rows_per_run(int T, long long M) {
+    const int most = T >= 64 ? 16 : (T >= 8 ? 4 : 1);
+    const int fit = M <= 2048 ? 1 : (M <= 4096 ? 2 : (M <= 32768 ? 4 : 16));
+    return std::min(most, fit);
+}
 
 kr_gemm_args gemm_args(const kr_half* A, int M, int K, const void* Wt, int N, void* out,
                        const kr_half* res = nullptr, const kr_half* gate = nullptr,
@@ -705,7 +718,7 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     a.state = Hm(st.att_xx);
     a.B = B;
     a.T = T;
-    a.run = rows_per_run(T);
+    a.run = rows_per_run(T, M);
     a.frag = fr ? 1 : 0;
     set_embed(a, e, x);
     // stepped: LN1 stages the int8 K, V, R and output-projection weights in
@@ -877,7 +890,7 @@ int layer_forward(const kr_layer_weights& L, int C, int F, kr_half* x, int B, in
     a.state = Hm(st.att_xx);
     a.B = B;
     a.T = T;
-    a.run = rows_per_run(T);
+    a.run = rows_per_run(T, M);
     a.frag = fr ? 1 : 0;
     set_embed(a, e, x);
     KR_TRY(ph.mark(0));
