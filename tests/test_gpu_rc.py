@@ -219,3 +219,24 @@ def test_compression_makes_progress():
     assert len(bits) < N // 4, len(bits)
     assert bits == orc.encode(cdf, sym)
     np.testing.assert_array_equal(krunch_ac.decode(bits, cdf), sym)
+
+
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 129, 1000])
+def test_wave_encoder_batches_and_pending_runs(N):
+    """The encoder takes 64 symbols at a time. Streams of ordinary symbols, of
+    one symbol whose interval [1/4, 3/4) emits nothing and only adds pending
+    bits (past 256 of them carried into a batch the bits go out serially), and
+    a mix, at lengths around a batch, in one call and in three: bytes and
+    state as the oracle's."""
+    q = 1 << 22
+    cdf3 = np.array([0, q, 3 * q, 4 * q], dtype=np.uint32)
+    rng = np.random.default_rng(N)
+    mixes = [rng.integers(0, 3, N), np.ones(N, dtype=np.int64),
+             np.where(rng.random(N) < 0.02, rng.integers(0, 3, N), 1)]
+    mixes.append(np.concatenate([np.ones(N - N // 4, dtype=np.int64), rng.integers(0, 3, N // 4)]))
+    for sym in mixes:
+        sym = sym.astype(np.int32)
+        cdf = np.tile(cdf3, (N, 1))
+        ref = orc.encode(cdf, sym)
+        assert _gpu_encode(cdf, sym) == ref
+        assert _gpu_encode(cdf, sym, chunks=min(3, N)) == ref
