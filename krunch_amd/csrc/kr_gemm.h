@@ -84,6 +84,14 @@ __host__ __device__ inline long long kr_frag_rows(long long R) { return (R + 15)
 // which also reads and writes fragment-packed operands.
 #define KR_GEMM_SMALL_M 512
 #define KR_GEMM_SMALL_MAX_N 16384
+// Fragment-packed products of more rows than that, up to this many, take the
+// register-fed kernel of kr_mid.hip. Measured on MI355X (one layer, us, tile
+// kernel / register-fed): fp16 157.6 / 155.7 at 2200 rows, 163.6 / 163.3 at
+// 2400, 178.7 / 194.5 at 2700; w8a8, with half the operand bytes, 119.3 /
+// 115.5 at 1500, 126.1 / 127.8 at 1800 (kr_layer.hip asks for fragment-packed
+// operands up to these limits).
+#define KR_GEMM_MID_M 2304
+#define KR_GEMM_MID_M_I8 1664
 
 // Up to three products with the same M and K in one launch.
 struct kr_gemm_multi {
@@ -159,6 +167,10 @@ int kr_gemm_head_big(const kr_half* A, long long lda, const kr_half* Wt, long lo
 // steps, 16-byte aligned operand rows, and N * (W^T row bytes) < 2^31.
 int kr_gemm_launch_wide(const kr_gemm_args& g, int epilogue, hipStream_t stream);
 
+
+// Up to three fragment-packed products that share M and K (and the operand
+// type), any M, in one launch (kr_mid.hip).
+int kr_gemm_launch_mid(const kr_gemm_multi& mj, hipStream_t stream);
 
 // Per-row symmetric int8 quantisation of an fp16 [M, K] matrix (kr_quant.hip).
 int kr_impl_quantize_rows(const void* x, long long ldx, int M, int K, void* q, float* scales,

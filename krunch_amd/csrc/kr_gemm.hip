@@ -1235,6 +1235,12 @@ int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* eps, int njobs, hi
     }
     if (M == 0) return KR_OK;
     const bool small = M <= KR_GEMM_SMALL_M && same && small_n;
+    if (M > KR_GEMM_SMALL_M && M <= (i8 ? KR_GEMM_MID_M_I8 : KR_GEMM_MID_M) && same && frag && !qa) {
+        kr_gemm_multi mj{};
+        mj.njobs = njobs;
+        for (int j = 0; j < njobs; j++) { mj.job[j] = jobs[j]; mj.ep[j] = eps[j]; }
+        return kr_gemm_launch_mid(mj, s);
+    }
     KR_REQUIRE(small || !any_frag, "gemm: fragment-packed operands need the small-M path "
                "(M <= %d, N < %d, one M/K/layout per launch)", KR_GEMM_SMALL_M, KR_GEMM_SMALL_MAX_N);
     if (small) {

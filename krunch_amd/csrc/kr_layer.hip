@@ -569,6 +569,18 @@ bool use_fragments_q8(const kr_layer_q8& Q, long long M) {
            Q.fR.qf;
 }
 
+// Above that, up to KR_GEMM_MID_M rows (w8a8 KR_GEMM_MID_M_I8), the products
+// read fragment-packed operands as well, in the register-fed kernel of
+// kr_mid.hip.
+bool use_mid(const kr_layer_weights& L, long long M) {
+    return M > KR_GEMM_SMALL_M && M <= KR_GEMM_MID_M && L.Kf && L.Vf && L.Rf && L.Of && L.fKf &&
+           L.fVf && L.fRf;
+}
+bool use_mid_q8(const kr_layer_q8& Q, long long M) {
+    return M > KR_GEMM_SMALL_M && M <= KR_GEMM_MID_M_I8 && Q.K.qf && Q.V.qf && Q.R.qf && Q.O.qf &&
+           Q.fK.qf && Q.fV.qf && Q.fR.qf;
+}
+
 // Layer 0's LN1-mix can run in the previous decode kernel (kr_embed_mix)
 // when the layer is a stepped one on fragment-packed weights
 // (layer_step_fused, or layer_forward_q8's stepped path).
@@ -708,6 +720,7 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     const kr_layer_q8& Q = *L.q8;
     const int M = B * T, G = C / 256;
     const bool fr = use_fragments_q8(Q, M);
+    const bool mid = use_mid_q8(Q, M);      // fragment-packed, quantised by row kernels
     LnMixArgs a{};
     a.x = x;
     a.ln_w = H(L.ln1_w);
@@ -719,7 +732,7 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     a.B = B;
     a.T = T;
     a.run = rows_per_run(T, M);
-    a.frag = fr ? 1 : 0;
+    a.frag = fr || mid ? 1 : 0;
     set_embed(a, e, x);
     // stepped: LN1 stages the int8 K, V, R and output-projection weights in
     // their XCDs' L2, LN2 the value product's (as layer_step_fused does)
@@ -755,9 +768,9 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
         KR_TRY(ph.mark(2));
     } else {
         {
-            const kr_gemm_args jobs[3] = {gemm_q8(w.kx8, w.kxs, M, C, Q.K, C, w.k, fr),
-                                          gemm_q8(w.vx8, w.vxs, M, C, Q.V, C, w.v, fr),
-                                          gemm_q8(w.rx8, w.rxs, M, C, Q.R, C, w.r, fr)};
+            const kr_gemm_args jobs[3] = {gemm_q8(w.kx8, w.kxs, M, C, Q.K, C, w.k, fr || mid),
+                                          gemm_q8(w.vx8, w.vxs, M, C, Q.V, C, w.v, fr || mid),
+                                          gemm_q8(w.rx8, w.rxs, M, C, Q.R, C, w.r, fr || mid)};
             const int eps[3] = {KR_EP_F32, KR_EP_F32, KR_EP_SIGMOID};
             KR_TRY(kr_gemm_launch_multi(jobs, eps, 3, s));
         }
@@ -768,8 +781,8 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     if (fr) {
         KR_TRY(kr_gemm_launch(gemm_q8_q16(w.ry, M, C, Q.O, C, x, x), KR_EP_RESID, s));
     } else {
-        KR_TRY(kr_impl_quantize_rows(w.ry, C, M, C, w.ry8, w.rys, 0, s));
-        KR_TRY(kr_gemm_launch(gemm_q8(w.ry8, w.rys, M, C, Q.O, C, x, false, x), KR_EP_RESID, s));
+        KR_TRY(kr_impl_quantize_rows(w.ry, C, M, C, w.ry8, w.rys, mid ? 1 : 0, s));
+        KR_TRY(kr_gemm_launch(gemm_q8(w.ry8, w.rys, M, C, Q.O, C, x, mid, x), KR_EP_RESID, s));
     }
     KR_TRY(ph.mark(4));
     a.ln_w = H(L.ln2_w);
@@ -781,8 +794,8 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     KR_TRY(launch_ln_mix<2>(G, a, s));
     KR_TRY(ph.mark(5));
     {
-        kr_gemm_args jobs[2] = {gemm_q8(w.frx8, w.frxs, M, C, Q.fR, C, w.rf, fr),
-                                gemm_q8(w.fkx8, w.fkxs, M, C, Q.fK, F, w.kf, fr)};
+        kr_gemm_args jobs[2] = {gemm_q8(w.frx8, w.frxs, M, C, Q.fR, C, w.rf, fr || mid),
+                                gemm_q8(w.fkx8, w.fkxs, M, C, Q.fK, F, w.kf, fr || mid)};
         jobs[1].out_frag = fr ? 1 : 0;     // the value product's fp16 operand
         const int eps[2] = {KR_EP_SIGMOID, KR_EP_RELUSQ};
         KR_TRY(kr_gemm_launch_multi(jobs, eps, 2, s));
@@ -791,8 +804,8 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     if (fr) {
         KR_TRY(kr_gemm_launch(gemm_q8_q16(w.kf, M, F, Q.fV, C, x, x, w.rf), KR_EP_GATED, s));
     } else {
-        KR_TRY(kr_impl_quantize_rows(w.kf, F, M, F, w.kf8, w.kfs, 0, s));
-        KR_TRY(kr_gemm_launch(gemm_q8(w.kf8, w.kfs, M, F, Q.fV, C, x, false, x, w.rf),
+        KR_TRY(kr_impl_quantize_rows(w.kf, F, M, F, w.kf8, w.kfs, mid ? 1 : 0, s));
+        KR_TRY(kr_gemm_launch(gemm_q8(w.kf8, w.kfs, M, F, Q.fV, C, x, mid, x, w.rf),
                               KR_EP_GATED, s));
     }
     return ph.mark(7);
@@ -879,8 +892,8 @@ int layer_forward(const kr_layer_weights& L, int C, int F, kr_half* x, int B, in
                "fragment-packed weights (fp16 or w8a8)");
     if (L.q8) return layer_forward_q8(L, C, F, x, B, T, st, w, s, e, ph);
     const int M = B * T, G = C / 256;
-    const bool fr = use_fragments(L, M);
-    if (fr && T == 1) return layer_step_fused(L, C, F, x, B, st, w, s, e, ph);
+    const bool fr = use_fragments(L, M) || use_mid(L, M);
+    if (use_fragments(L, M) && T == 1) return layer_step_fused(L, C, F, x, B, st, w, s, e, ph);
     LnMixArgs a{};
     a.x = x;
     a.ln_w = H(L.ln1_w);

@@ -178,15 +178,27 @@ _WT_CACHE: dict = {}
 
 def _wt(W):
     """Transposed copy of a [K, N] weight, cached per live tensor object and version."""
+    return _wt_wf(W)[0]
+
+
+def _wt_wf(W, frag=False):
+    """The same with, on request, the fragment-packed copy that the layer's
+    products read (kept in the same entry; else None). frag needs K % 32 == 0."""
     key = id(W)
     hit = _WT_CACHE.get(key)
     if hit is None or hit[0]() is not W or hit[1] != W._version:
         K, N = W.shape
         wt = torch.empty((N, K), dtype=torch.float16, device=W.device)
         _lib.call("kr_transpose_f16", W.data_ptr(), N, K, N, wt.data_ptr(), K, _lib.stream_ptr())
-        hit = (weakref.ref(W, lambda _r, k=key: _WT_CACHE.pop(k, None)), W._version, wt)
+        hit = (weakref.ref(W, lambda _r, k=key: _WT_CACHE.pop(k, None)), W._version, wt, None)
         _WT_CACHE[key] = hit
-    return hit[2]
+    if frag and hit[3] is None:
+        N, K = hit[2].shape
+        wf = torch.empty(_lib.lib().kr_fragment_bytes(N, K), dtype=torch.uint8, device=W.device)
+        _lib.call("kr_pack_fragments", hit[2].data_ptr(), K, N, K, wf.data_ptr(), _lib.stream_ptr())
+        hit = hit[:3] + (wf,)
+        _WT_CACHE[key] = hit
+    return hit[2:]
 
 
 def det_matmul(x, W, out_dtype=None):
@@ -231,16 +243,17 @@ def _layer_struct(x, att_xx, aa, bb, pp, ffn_xx, ln1_w, ln1_b, tm_k, tm_v, tm_r,
     def wt(m, k, n):
         _cuda(m, torch.float16, "weight")
         _check(tuple(m.shape) == (k, n), f"weight must be [{k}, {n}], got {tuple(m.shape)}")
-        t = _wt(m)
-        keep.append(t)
-        return t.data_ptr()
+        t = _wt_wf(m, frag=True)
+        keep.extend(t)
+        return t[0].data_ptr(), t[1].data_ptr()
 
     L = _lib.KrLayerWeights()
     L.ln1_w, L.ln1_b, L.tm_k, L.tm_v, L.tm_r = map(h, (ln1_w, ln1_b, tm_k, tm_v, tm_r))
     L.decay, L.first = f32(time_decay), f32(time_first)
-    L.Kt, L.Vt, L.Rt, L.Ot = (wt(m, C, C) for m in (Kw, Vw, Rw, Ow))
+    (L.Kt, L.Kf), (L.Vt, L.Vf), (L.Rt, L.Rf), (L.Ot, L.Of) = (wt(m, C, C) for m in (Kw, Vw, Rw, Ow))
     L.ln2_w, L.ln2_b, L.ftm_k, L.ftm_r = map(h, (ln2_w, ln2_b, ffn_tm_k, ffn_tm_r))
-    L.fKt, L.fVt, L.fRt = wt(ffn_Kw, C, F), wt(ffn_Vw, F, C), wt(ffn_Rw, C, C)
+    (L.fKt, L.fKf), (L.fVt, L.fVf), (L.fRt, L.fRf) = (wt(ffn_Kw, C, F), wt(ffn_Vw, F, C),
+                                                      wt(ffn_Rw, C, C))
     for t, dt, n in ((att_xx, torch.float16, "att_xx"), (aa, torch.float32, "aa"),
                      (bb, torch.float32, "bb"), (pp, torch.float32, "pp"),
                      (ffn_xx, torch.float16, "ffn_xx")):
