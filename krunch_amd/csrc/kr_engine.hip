@@ -223,6 +223,10 @@ int kr_decode_run(const kr_model_weights* m, int B, void* state, int32_t* syms, 
             for (int g = 0; g < ng; g++) KR_TRY(decode_step(grp[g], s));
         return KR_OK;
     }
+    // the steps run as graphs on the caller's stream and are waited for here
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
+        return kr_fail(KR_EHIP, "kr_decode_run: use_graph on a stream that is being captured");
     // Warm per-V caches (CDF summation plan) outside the capture: a
     // zero-row launch builds the plan without running a kernel.
     KR_TRY(kr_probs_to_cdf(reinterpret_cast<const float*>(logits), 0, m->V, m->V, ac_states,
@@ -241,7 +245,7 @@ int kr_decode_run(const kr_model_weights* m, int B, void* state, int32_t* syms, 
     // Several groups: one graph per step, the groups as independent branches
     // (fork/join through events), so their latency-bound kernels overlap.
     hipStream_t cap[16] = {};
-    hipEvent_t ev[18] = {};
+    hipEvent_t ev[16] = {};
     hipGraph_t graph[2] = {};
     hipGraphExec_t exec[2] = {};
     int rc = KR_OK;
@@ -266,7 +270,7 @@ int kr_decode_run(const kr_model_weights* m, int B, void* state, int32_t* syms, 
     for (int g = 0; g < ng; g++)
         if ((e = hipStreamCreateWithFlags(&cap[g], hipStreamNonBlocking)) != hipSuccess)
             return hip_fail(e, "stream");
-    for (int i = 0; i < ng + 2; i++)
+    for (int i = 0; i < ng; i++)
         if ((e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming)) != hipSuccess)
             return hip_fail(e, "event");
     if (fold) {
@@ -276,9 +280,12 @@ int kr_decode_run(const kr_model_weights* m, int B, void* state, int32_t* syms, 
                 hipSuccess)
             return hip_fail(e, "layer-0 mix arguments");
     }
-    // ev[0]: caller -> capture stream; ev[1]: fork; ev[2+g]: join of group g; ev[ng+1] reused at the end
-    if ((e = hipEventRecord(ev[0], s)) != hipSuccess) return hip_fail(e, "record");
-    if ((e = hipStreamWaitEvent(cap[0], ev[0], 0)) != hipSuccess) return hip_fail(e, "wait");
+    // The cap streams only record: the graphs run on the caller's stream. On
+    // a stream of their own they took a hardware queue beside the caller's,
+    // whose wait for the last step's event then slowed every dispatch: 430 us
+    // per step against 365 at B = 17 on MI355X, in whichever calls the
+    // runtime gave the two streams different queues (about four of five).
+    // ev[0]: fork; ev[g]: join of group g.
     // graph i: step kind 0 (unfolded, or a folded run's first step) or 1 (a
     // folded run's later steps)
     auto capture = [&](int i) -> int {
@@ -286,16 +293,16 @@ int kr_decode_run(const kr_model_weights* m, int B, void* state, int32_t* syms, 
         if ((ce = hipStreamBeginCapture(cap[0], hipStreamCaptureModeThreadLocal)) != hipSuccess)
             return hip_fail(ce, "begin capture");
         capturing = true;
-        if ((ce = hipEventRecord(ev[1], cap[0])) != hipSuccess) return hip_fail(ce, "fork record");
+        if ((ce = hipEventRecord(ev[0], cap[0])) != hipSuccess) return hip_fail(ce, "fork record");
         for (int g = 1; g < ng; g++)
-            if ((ce = hipStreamWaitEvent(cap[g], ev[1], 0)) != hipSuccess) return hip_fail(ce, "fork wait");
+            if ((ce = hipStreamWaitEvent(cap[g], ev[0], 0)) != hipSuccess) return hip_fail(ce, "fork wait");
         if (fold) rc = decode_step(grp[0], cap[0], i == 0 ? dev_first : dev_next, i == 1);
         else
             for (int g = 0; g < ng && rc == KR_OK; g++) rc = decode_step(grp[g], cap[g]);
         if (rc) { cleanup(); return rc; }
         for (int g = 1; g < ng; g++) {
-            if ((ce = hipEventRecord(ev[1 + g], cap[g])) != hipSuccess) return hip_fail(ce, "join record");
-            if ((ce = hipStreamWaitEvent(cap[0], ev[1 + g], 0)) != hipSuccess) return hip_fail(ce, "join wait");
+            if ((ce = hipEventRecord(ev[g], cap[g])) != hipSuccess) return hip_fail(ce, "join record");
+            if ((ce = hipStreamWaitEvent(cap[0], ev[g], 0)) != hipSuccess) return hip_fail(ce, "join wait");
         }
         ce = hipStreamEndCapture(cap[0], &graph[i]);
         capturing = false;
@@ -307,11 +314,10 @@ int kr_decode_run(const kr_model_weights* m, int B, void* state, int32_t* syms, 
     if (capture(0)) return rc;
     if (fold && n_steps > 1 && capture(1)) return rc;
     for (int i = 0; i < n_steps; i++)
-        if ((e = hipGraphLaunch(exec[fold && i > 0 ? 1 : 0], cap[0])) != hipSuccess)
+        if ((e = hipGraphLaunch(exec[fold && i > 0 ? 1 : 0], s)) != hipSuccess)
             return hip_fail(e, "graph launch");
-    if ((e = hipEventRecord(ev[ng + 1], cap[0])) != hipSuccess) return hip_fail(e, "record");
-    if ((e = hipStreamWaitEvent(s, ev[ng + 1], 0)) != hipSuccess) return hip_fail(e, "wait");
-    if ((e = hipStreamSynchronize(cap[0])) != hipSuccess) return hip_fail(e, "sync");
+    // the graphs go with this call, so it waits for them
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "sync");
     cleanup();
     return KR_OK;
 }
