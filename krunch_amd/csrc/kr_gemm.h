@@ -93,12 +93,22 @@ __host__ __device__ inline long long kr_frag_rows(long long R) { return (R + 15)
 #define KR_GEMM_MID_M 2304
 #define KR_GEMM_MID_M_I8 1664
 
+// A row copy that rides along in a small-M product launch (8-byte units,
+// 8-byte aligned): the carried rows a fused LN-mix left beside the state it
+// read (kr_step.hip).
+struct kr_row_copy {
+    const uint2* src;
+    uint2* dst;
+    int n;
+};
+
 // Up to three products with the same M and K in one launch.
 struct kr_gemm_multi {
     kr_gemm_args job[KR_GEMM_MAX_JOBS];
     int ep[KR_GEMM_MAX_JOBS];
     int tiles[KR_GEMM_MAX_JOBS];
     int njobs;
+    kr_row_copy copy;          // n = 0: none
     // decode-step timing (null otherwise): wave w of workgroup b stores its
     // start and end times (the 100 MHz steady counter) at stamps[16 b + w]
     unsigned long long* stamps;
@@ -111,7 +121,9 @@ struct kr_gemm_multi {
 //   acc = P_0; acc = acc + P_1; ...; acc = acc + P_{S-1}   (fp32 adds, in order),
 // then the epilogue. A row therefore gets identical bits for any M. The int8
 // path accumulates exactly in int32, so any order gives the same bits.
-int kr_gemm_launch(const kr_gemm_args& g, int epilogue, hipStream_t stream);
+// copy (nullable): done in the same launch; fragment-packed small-M products only.
+int kr_gemm_launch(const kr_gemm_args& g, int epilogue, hipStream_t stream,
+                   const kr_row_copy* copy = nullptr);
 
 // Kernel timing for the decode-step profiler: the next small-M panel launch
 // on this host thread (kr_gemm_launch / kr_gemm_launch_multi choosing
@@ -139,7 +151,7 @@ int kr_gemm_timed_launch_taken();
 int kr_gemm_panel_ns(const kr_gemm_args* jobs, int njobs);
 
 int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* epilogues, int njobs,
-                         hipStream_t stream);
+                         hipStream_t stream, const kr_row_copy* copy = nullptr);
 
 // The head (logits = fp16(LN_out(x) @ head)) has a reduction contract of
 // its own, which the two head kernels below share and no other product uses:

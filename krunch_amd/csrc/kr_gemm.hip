@@ -634,6 +634,16 @@ __global__ void __launch_bounds__(MAXT) gemm_panel_kernel(kr_gemm_multi mj) {
             }
         }
     }
+    // ---- row copy: this thread's first unit fetched here, stored at the end
+    const int cp0 = bid * (int)blockDim.x + (int)threadIdx.x;
+    uint2 cp_v;
+    if (FRAG && cp0 < mj.copy.n) cp_v = mj.copy.src[cp0];
+    auto copy_rows = [&]() {
+        if (!FRAG || cp0 >= mj.copy.n) return;
+        mj.copy.dst[cp0] = cp_v;
+        for (int u = cp0 + (int)(gridDim.x * blockDim.x); u < mj.copy.n; u += (int)(gridDim.x * blockDim.x))
+            mj.copy.dst[u] = mj.copy.src[u];
+    };
     __builtin_amdgcn_sched_barrier(0);     // loads in flight before the MFMAs
 
     // ---- QA: row maxima over all slices, then this slice rounded to int8
@@ -786,6 +796,7 @@ __global__ void __launch_bounds__(MAXT) gemm_panel_kernel(kr_gemm_multi mj) {
             if constexpr (I8) epilogue(t, t, dequant(t, p[t / NS][t % NS]));
             else epilogue(t, t, p[t / NS][t % NS]);
         }
+        copy_rows();
         stamp_end();
         return;
     }
@@ -801,6 +812,7 @@ __global__ void __launch_bounds__(MAXT) gemm_panel_kernel(kr_gemm_multi mj) {
         if constexpr (I8) epilogue(t, e, dequant(t, acc));
         else epilogue(t, e, acc);
     }
+    copy_rows();
     stamp_end();
 }
 
@@ -1214,7 +1226,8 @@ int kr_gemm_panel_ns(const kr_gemm_args* jobs, int njobs) {
     return choose_small_shape(mj).NS;
 }
 
-int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* eps, int njobs, hipStream_t s) {
+int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* eps, int njobs, hipStream_t s,
+                         const kr_row_copy* copy) {
     KR_REQUIRE(njobs >= 1 && njobs <= KR_GEMM_MAX_JOBS, "gemm: bad job count %d", njobs);
     for (int j = 0; j < njobs; j++) {
         const int rc = check_args(jobs[j], eps[j]);
@@ -1234,6 +1247,7 @@ int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* eps, int njobs, hi
         any_frag = any_frag || jobs[j].a_frag || jobs[j].out_frag;
     }
     if (M == 0) return KR_OK;
+    KR_REQUIRE(!copy || (M <= KR_GEMM_SMALL_M && frag), "gemm: a row copy needs the small-M fragment path");
     const bool small = M <= KR_GEMM_SMALL_M && same && small_n;
     if (M > KR_GEMM_SMALL_M && M <= (i8 ? KR_GEMM_MID_M_I8 : KR_GEMM_MID_M) && same && frag && !qa) {
         kr_gemm_multi mj{};
@@ -1248,6 +1262,7 @@ int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* eps, int njobs, hi
         kr_gemm_multi mj{};
         mj.njobs = njobs;
         for (int j = 0; j < njobs; j++) { mj.job[j] = jobs[j]; mj.ep[j] = eps[j]; }
+        if (copy) mj.copy = *copy;
         if (qa) return launch_small<true, true, true>(mj, s);
         if (frag) return i8 ? launch_small<true, true>(mj, s) : launch_small<true, false>(mj, s);
         // row-major A: fragment weights are not used, the row-major copy must exist
@@ -1288,8 +1303,8 @@ int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* eps, int njobs, hi
     return KR_OK;
 }
 
-int kr_gemm_launch(const kr_gemm_args& g, int ep, hipStream_t s) {
-    return kr_gemm_launch_multi(&g, &ep, 1, s);
+int kr_gemm_launch(const kr_gemm_args& g, int ep, hipStream_t s, const kr_row_copy* copy) {
+    return kr_gemm_launch_multi(&g, &ep, 1, s, copy);
 }
 
 extern "C" {
@@ -1369,6 +1384,7 @@ int kr_det_matmul_packed_multi(const kr_packed_job* jobs, int n_jobs, int M, int
 int kr_det_matmul_packed(const uint16_t* xf, int M, int K, const uint16_t* Wf, int N, void* out,
                          long long ldo, int epilogue, const uint16_t* res, const uint16_t* gate,
                          int out_packed, void* stream) {
+    KR_REQUIRE(M <= KR_GEMM_SMALL_M, "kr_det_matmul_packed: M=%d (M <= %d)", M, KR_GEMM_SMALL_M);
     kr_gemm_args g{};
     g.A = reinterpret_cast<const kr_half*>(xf);
     g.lda = K;

@@ -22,6 +22,7 @@
 #include "kr_math.h"
 #include "kr_model.h"
 #include "kr_rowops.h"
+#include "kr_step.h"
 #include "kr_wave.h"
 #include "kr_wkv.h"
 
@@ -714,6 +715,62 @@ PrefetchSet att_stage_set(const kr_layer_weights& L, int C, int M, const Work& w
     return pf;
 }
 
+// A stepped layer with LN1-mix inside the K, V, R + WKV launch and LN2-mix
+// inside the channel mix's R + K launch (kr_step.hip): four launches. The
+// carried rows wait in the workspace's kx and fkx rows, which such a layer
+// does not use otherwise, until the next product copies them to the state.
+// Not for layer 0 of a forward from token ids, whose LN1-mix gathers the
+// embedding (or ran in the decode kernel), and not while that step's panel
+// products are timed (kr_step_timing's phases name separate launches).
+bool use_step_fused(int M, int F, bool i8, const EmbedSrc* e, const Phases& ph) {
+    return M <= (i8 ? KR_STEP_FUSE_M_I8 : KR_STEP_FUSE_M) && F % 256 == 0 && !e && !ph.stamps;
+}
+
+kr_step_kvr step_kvr_args(const kr_layer_weights& L, const kr_half* x, int M, const kr_layer_state& st,
+                          const Work& w) {
+    kr_step_kvr a{};
+    a.ln = kr_step_ln{x, H(L.ln1_w), H(L.ln1_b), {H(L.tm_k), H(L.tm_v), H(L.tm_r)},
+                      H(st.att_xx), w.kx};
+    a.Wf[0] = H(L.Kf); a.Wf[1] = H(L.Vf); a.Wf[2] = H(L.Rf);
+    if (L.q8) {
+        const kr_layer_q8& Q = *L.q8;
+        a.Wf[0] = H(Q.K.qf); a.Wf[1] = H(Q.V.qf); a.Wf[2] = H(Q.R.qf);
+        a.sw[0] = Q.K.scale; a.sw[1] = Q.V.scale; a.sw[2] = Q.R.scale;
+    }
+    a.decay = L.decay;
+    a.first = L.first;
+    a.aa = st.aa;
+    a.bb = st.bb;
+    a.pp = st.pp;
+    a.ry = w.ry;
+    a.M = M;
+    return a;
+}
+
+kr_step_rk step_rk_args(const kr_layer_weights& L, const kr_half* x, int M, int F,
+                        const kr_layer_state& st, const Work& w) {
+    kr_step_rk a{};
+    a.ln = kr_step_ln{x, H(L.ln2_w), H(L.ln2_b), {H(L.ftm_k), H(L.ftm_r), nullptr},
+                      H(st.ffn_xx), w.fkx};
+    a.WfR = H(L.fRf);
+    a.WfK = H(L.fKf);
+    if (L.q8) {
+        a.WfR = H(L.q8->fR.qf);
+        a.WfK = H(L.q8->fK.qf);
+        a.swR = L.q8->fR.scale;
+        a.swK = L.q8->fK.scale;
+    }
+    a.rf = w.rf;
+    a.kf = w.kf;
+    a.F = F;
+    a.M = M;
+    return a;
+}
+
+kr_row_copy carried_rows(const kr_half* pend, void* state, int M, int C) {
+    return kr_row_copy{reinterpret_cast<const uint2*>(pend), static_cast<uint2*>(state), M * C / 4};
+}
+
 int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B, int T,
                      const kr_layer_state& st, const Work& w, hipStream_t s,
                      const EmbedSrc* e, const Phases& ph) {
@@ -721,6 +778,21 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     const int M = B * T, G = C / 256;
     const bool fr = use_fragments_q8(Q, M);
     const bool mid = use_mid_q8(Q, M);      // fragment-packed, quantised by row kernels
+    if (fr && T == 1 && use_step_fused(M, F, true, e, ph)) {
+        KR_TRY(ph.mark(0));
+        KR_TRY(ph.mark(1));
+        KR_TRY(kr_step_launch_kvr(C, true, step_kvr_args(L, x, M, st, w), s));
+        KR_TRY(ph.mark(2));
+        KR_TRY(ph.mark(3));
+        const kr_row_copy att = carried_rows(w.kx, st.att_xx, M, C), ffn = carried_rows(w.fkx, st.ffn_xx, M, C);
+        KR_TRY(kr_gemm_launch(gemm_q8_q16(w.ry, M, C, Q.O, C, x, x), KR_EP_RESID, s, &att));
+        KR_TRY(ph.mark(4));
+        KR_TRY(ph.mark(5));
+        KR_TRY(kr_step_launch_rk(C, true, step_rk_args(L, x, M, F, st, w), s));
+        KR_TRY(ph.mark(6));
+        KR_TRY(kr_gemm_launch(gemm_q8_q16(w.kf, M, F, Q.fV, C, x, x, w.rf), KR_EP_GATED, s, &ffn));
+        return ph.mark(7);
+    }
     LnMixArgs a{};
     a.x = x;
     a.ln_w = H(L.ln1_w);
@@ -813,12 +885,27 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
 
 // Stepped (T = 1) fp16 layer with fragment-packed weights: LN1-mix, the
 // K, V, R products fused with WKV, the output projection, LN2-mix and the
-// channel mix (six launches).
+// channel mix (six launches; four at few streams, use_step_fused).
 
 int layer_step_fused(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
                      const kr_layer_state& st, const Work& w, hipStream_t s,
                      const EmbedSrc* e, const Phases& ph) {
     const int M = B, G = C / 256;
+    if (use_step_fused(M, F, false, e, ph)) {
+        KR_TRY(ph.mark(0));
+        KR_TRY(ph.mark(1));
+        KR_TRY(kr_step_launch_kvr(C, false, step_kvr_args(L, x, M, st, w), s));
+        KR_TRY(ph.mark(2));
+        KR_TRY(ph.mark(3));
+        const kr_row_copy att = carried_rows(w.kx, st.att_xx, M, C), ffn = carried_rows(w.fkx, st.ffn_xx, M, C);
+        KR_TRY(kr_gemm_launch(gemm_args(w.ry, M, C, L.Ot, C, x, x, nullptr, L.Of, true), KR_EP_RESID, s, &att));
+        KR_TRY(ph.mark(4));
+        KR_TRY(ph.mark(5));
+        KR_TRY(kr_step_launch_rk(C, false, step_rk_args(L, x, M, F, st, w), s));
+        KR_TRY(ph.mark(6));
+        KR_TRY(kr_gemm_launch(gemm_args(w.kf, M, F, L.fVt, C, x, x, w.rf, L.fVf, true), KR_EP_GATED, s, &ffn));
+        return ph.mark(7);
+    }
     // Weights the next products read, staged into their XCDs' L2 by the
     // LN-mix launches (which wait on memory latency, not bandwidth): LN1 stages
     // K, V, R and the output projection, LN2 the channel-mix value product.

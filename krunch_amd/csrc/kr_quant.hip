@@ -117,6 +117,8 @@ int kr_det_matmul_i8(const int8_t* xq, const float* sa, int M, int K, const int8
                      const float* sw, int N, void* out, long long ldo, int epilogue,
                      const uint16_t* res, const uint16_t* gate, int packed, void* stream) {
     KR_REQUIRE(packed >= 0 && packed <= 2, "kr_det_matmul_i8: packed must be 0, 1 or 2");
+    KR_REQUIRE(!packed || M <= KR_GEMM_SMALL_M, "kr_det_matmul_i8: packed operands need M <= %d (M=%d)",
+               KR_GEMM_SMALL_M, M);
     kr_gemm_args g{};
     g.A = reinterpret_cast<const kr_half*>(xq);
     g.lda = K;
