@@ -160,7 +160,7 @@ int kr_compress_window(const kr_model_weights* m, const int32_t* inputs, const i
         const int n = (int)((M - r0) < head_rows ? (M - r0) : head_rows);
         const void* xr = static_cast<const char*>(x) + (size_t)r0 * m->C * 2;
         void* xnr = static_cast<char*>(xn) + (size_t)r0 * m->C * 2;
-        KR_TRY(kr_impl_head(m, xr, n, xnr, logits, ld, s, head_rows % 16 == 0));
+        KR_TRY(kr_impl_head(m, xr, n, xnr, logits, ld, s, head_rows % 16 == 0 || M <= head_rows));
         KR_TRY(kr_softmax_cdf_pairs(reinterpret_cast<const uint16_t*>(logits), n, m->V, ld,
                                     targets + r0, pairs + 2 * r0, cdf_precision, stream));
     }

@@ -168,6 +168,10 @@ int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* epilogues, int njo
 bool kr_gemm_head_small_ok(int M, int N, int K);
 int kr_gemm_head_small(const kr_half* Af, const kr_half* Wf, int M, int N, int K, kr_half* out,
                        long long ldo, hipStream_t stream);
+// The same for M > 512 (kr_head.hip): any ldo >= N below 2^24.
+bool kr_gemm_head_rows_ok(int M, int N, int K);
+int kr_gemm_head_rows(const kr_half* Af, const kr_half* Wf, int M, int N, int K, kr_half* out,
+                      long long ldo, hipStream_t stream);
 // The same product for any M: A [M, K] row-major (row stride lda), W^T [N, K]
 // row-major (row stride ldw); K % 64 == 0, lda and ldw multiples of 8,
 // A and Wt 16-byte aligned, N * ldw * 2 < 2^31.

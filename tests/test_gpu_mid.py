@@ -5,7 +5,7 @@ contract makes them equal bit for bit, state included."""
 import pytest
 import torch
 
-from krunch_amd import cpp_path, krunch_ac_hip, synthetic
+from krunch_amd import _lib, cpp_path, krunch_ac_hip, synthetic
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +55,33 @@ def test_layer_op_repacks_a_changed_weight():
     after = step(mats)
     assert not torch.equal(before, after)
     assert torch.equal(after, step([m.clone() for m in mats]))
+
+
+# rows past the decode head's 512, at and around its 256-row groups and
+# 16-row blocks; row strides of every alignment; column counts with and
+# without a last partial block, fewer blocks than a run's pipeline, and
+# widths with 8, 16 and 24 fragments per row
+@pytest.mark.parametrize("C,V,M,ld", [(768, 1000, 528, 1000), (768, 1003, 513 + 15, 1003), (768, 50277, 784, 50277),
+                                      (768, 1001, 1040, 1002), (512, 777, 2064, 779), (256, 40, 768, 41),
+                                      (768, 3, 544, 5), (256, 5000, 8208, 5000), (512, 2000, 512 + 256, 2000)])
+def test_head_rows_equals_single_blocks(C, V, M, ld):
+    """The head over many rows against the same rows 256 at a time (the decode
+    head): the one-chain contract makes them equal bit for bit. Nothing is
+    written past a row's V columns."""
+    w = synthetic.make_weights(n_layer=1, C=C, F=4 * C, V=V, seed=C + V)
+    P = cpp_path.init_weights(w, "cuda")["prepared"]
+    try:
+        g = torch.Generator(device="cuda").manual_seed(M)
+        x = torch.randn((M, C), generator=g, device="cuda").half()
+        xn = torch.empty_like(x)
+        s = _lib.stream_ptr()
+        got = torch.full((M, ld), 7.0, dtype=torch.float16, device="cuda")
+        ref = got.clone()
+        _lib.call("kr_head_logits", P.ptr, x.data_ptr(), M, xn.data_ptr(), got.data_ptr(), ld, s)
+        for r in range(0, M, 256):
+            n = min(256, M - r)
+            _lib.call("kr_head_logits", P.ptr, x[r:].data_ptr(), n, xn.data_ptr(), ref[r:].data_ptr(), ld, s)
+        assert torch.equal(got, ref)
+        assert bool((got[:, V:] == 7.0).all())
+    finally:
+        cpp_path.release_weights(w)
