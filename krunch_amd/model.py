@@ -157,6 +157,23 @@ class State:
         _lib.call("kr_state_init", self.buf.data_ptr(), self.n_layer, self.B, self.C,
                   _lib.stream_ptr())
 
+    def first(self, n: int) -> "State":
+        """A state of its own with the first n streams of this one."""
+        out = object.__new__(State)
+        out.n_layer, out.B, out.C, out.device = self.n_layer, n, self.C, self.device
+        out.buf = torch.empty(_lib.lib().kr_state_bytes(self.n_layer, n, self.C), dtype=torch.uint8,
+                              device=self.device)
+        for a, b in zip(self._parts(), out._parts()):
+            b.copy_(a[:, :, :n])
+        return out
+
+    def _parts(self):
+        """All layers' [att_xx, ffn_xx] and [aa, bb, pp], as views over the streams."""
+        n = 4 * self.B * self.C
+        raw = self.buf[:4 * n * self.n_layer].view(self.n_layer, 4 * n)
+        return (raw[:, :n].view(torch.float16).view(self.n_layer, 2, self.B, self.C),
+                raw[:, n:].view(torch.float32).view(self.n_layer, 3, self.B, self.C))
+
     def _layer(self, i):
         B, C = self.B, self.C
         per = B * C * 16
