@@ -183,20 +183,23 @@ def _wt(W):
 
 def _wt_wf(W, frag=False):
     """The same with, on request, the fragment-packed copy that the layer's
-    products read (kept in the same entry; else None). frag needs K % 32 == 0."""
+    products read (kept in the same entry; else None). frag needs K % 32 == 0.
+    Copies made while the stream is capturing are written when the graph runs,
+    not now, so they serve that call only."""
     key = id(W)
     hit = _WT_CACHE.get(key)
+    known = hit
     if hit is None or hit[0]() is not W or hit[1] != W._version:
         K, N = W.shape
         wt = torch.empty((N, K), dtype=torch.float16, device=W.device)
         _lib.call("kr_transpose_f16", W.data_ptr(), N, K, N, wt.data_ptr(), K, _lib.stream_ptr())
         hit = (weakref.ref(W, lambda _r, k=key: _WT_CACHE.pop(k, None)), W._version, wt, None)
-        _WT_CACHE[key] = hit
     if frag and hit[3] is None:
         N, K = hit[2].shape
         wf = torch.empty(_lib.lib().kr_fragment_bytes(N, K), dtype=torch.uint8, device=W.device)
         _lib.call("kr_pack_fragments", hit[2].data_ptr(), K, N, K, wf.data_ptr(), _lib.stream_ptr())
         hit = hit[:3] + (wf,)
+    if hit is not known and not torch.cuda.is_current_stream_capturing():
         _WT_CACHE[key] = hit
     return hit[2:]
 

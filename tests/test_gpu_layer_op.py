@@ -1,0 +1,62 @@
+"""The layer op's weight copies (transposed and fragment-packed, kept per
+weight tensor): calls inside a stream capture."""
+import pytest
+import torch
+
+from krunch_amd import krunch_ac_hip as ops
+
+pytestmark = pytest.mark.gpu
+C, F = 256, 512
+SHAPES = ((C, C), (C, C), (C, C), (C, C), (C, F), (F, C), (C, C))
+
+
+def _inputs(B, T, seed):
+    g = torch.Generator().manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    return {"x": rnd(B, T, C).half().cuda(), "ln": [rnd(C).half().cuda() for _ in range(4)],
+            "tm": [torch.rand(C, generator=g).half().cuda() for _ in range(5)],
+            "decay": (-torch.rand(C, generator=g)).cuda(), "first": torch.zeros(C).cuda(),
+            "mats": [(0.05 * rnd(k, n)).half().cuda() for k, n in SHAPES]}
+
+
+def _state(B):
+    h = lambda: torch.zeros(B, C, dtype=torch.float16, device="cuda")
+    return [h(), *(torch.zeros(B, C, device="cuda") for _ in range(3)), h()]
+
+
+def _call(d, st, mats=None):
+    m = mats or d["mats"]
+    return ops.rwkv4_layer_step_cpp(d["x"], *st, *d["ln"][:2], *d["tm"][:3], d["decay"], d["first"],
+                                    *m[:4], *d["ln"][2:], *d["tm"][3:], *m[4:])
+
+
+# weights never seen before, and weights whose transposed copies det_matmul
+# made; a stepped call, a small and a mid-sized window
+@pytest.mark.parametrize("warm", [False, True])
+@pytest.mark.parametrize("B,T", [(3, 1), (2, 40), (2, 300)])
+def test_layer_captured_on_new_weights(B, T, warm):
+    """Copies made while a stream is capturing are written when the graph
+    runs, so they must not serve a call made before that."""
+    d = _inputs(B, T, 10 * B + T)
+    ref_st = _state(B)
+    ref = _call(d, ref_st, [m.clone() for m in d["mats"]])
+    if warm:
+        for m in d["mats"]:
+            ops.det_matmul(torch.zeros(1, m.shape[0], dtype=torch.float16, device="cuda"), m)
+    st = _state(B)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = _call(d, st)
+    eager_st = _state(B)
+    assert torch.equal(_call(d, eager_st), ref)
+    for a, b in zip(eager_st, ref_st):
+        assert torch.equal(a, b)
+    for _ in range(3):
+        for a, b in zip(st, _state(B)):
+            a.copy_(b)
+        graph.replay()
+        assert torch.equal(out, ref)
+        for a, b in zip(st, ref_st):
+            assert torch.equal(a, b)
+        assert torch.equal(_call(d, _state(B)), ref)
