@@ -141,7 +141,9 @@ int kr_embed(const kr_model_weights* m, const int32_t* ids, int M, void* x, void
 int kr_head_logits(const kr_model_weights* m, const void* x, int M, void* xn, void* logits,
                    long long ld, void* stream) {
     KR_REQUIRE(m && x && xn && logits && M >= 0 && ld >= m->V, "kr_head_logits: bad args");
-    return kr_impl_head(m, x, M, xn, logits, ld, kr_stream(stream), M % 16 == 0);
+    // fragment-packed rows are spread over their 16-row block, so only
+    // row-major LN_out can run in place
+    return kr_impl_head(m, x, M, xn, logits, ld, kr_stream(stream), M % 16 == 0 && xn != x);
 }
 
 int kr_compress_window(const kr_model_weights* m, const int32_t* inputs, const int32_t* targets,
