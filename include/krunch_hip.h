@@ -312,7 +312,8 @@ int kr_reset_phase_times(void);
  * the stepped decode. kr_step_timing(p) with p = 3 (ow_matmul_residual),
  * 5 (ffn_rk_matmul) or 6 (ffn_v_matmul_residual) times that phase's product
  * in every layer of every later decode step (kr_decode_step, kr_decode_run,
- * graph or eager): each of its waves stores its start and end on the GPU's
+ * graph or eager; at few streams phase 5's launch holds the LN2-mix too): each
+ * of its waves stores its start and end on the GPU's
  * 100 MHz steady counter (a vector store per wave, also at every replay of a
  * captured graph), and in eager steps the launch goes through
  * hipExtLaunchKernel with two HIP events that take its dispatch's start and

@@ -127,10 +127,10 @@ int kr_gemm_launch(const kr_gemm_args& g, int epilogue, hipStream_t stream,
 
 // Kernel timing for the decode-step profiler: the next small-M panel launch
 // on this host thread (kr_gemm_launch / kr_gemm_launch_multi choosing
-// gemm_panel_kernel) with at most max_groups workgroups gets `stamps`
-// (2 x KR_STAMP_WAVES x max_groups u64, see kr_gemm_multi) and stores each
-// wave's start and end times there, also when it is captured in a graph
-// (then at every replay). Arm with a buffer, disarm with nullptr.
+// gemm_panel_kernel, or kr_step_launch_rk) with at most max_groups workgroups
+// gets `stamps` (2 x KR_STAMP_WAVES x max_groups u64, see kr_gemm_multi) and
+// stores each wave's start and end times there, also when it is captured in a
+// graph (then at every replay). Arm with a buffer, disarm with nullptr.
 // kr_gemm_timed_launch_taken(): the grid size of the panel launch that took
 // the buffer since it was armed; 0 if none came; minus the grid size if one
 // came with more than max_groups workgroups (it ran untimed).
@@ -141,6 +141,13 @@ constexpr int KR_STAMP_WAVES = 16;
 void kr_gemm_time_next_panel(unsigned long long* stamps, int max_groups,
                              hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 int kr_gemm_timed_launch_taken();
+// What a panel launch of `groups` workgroups of `waves` waves takes of that
+// (which disarms it); nulls when nothing is armed or the launch does not fit.
+struct kr_panel_timing {
+    unsigned long long* stamps;
+    hipEvent_t start, stop;
+};
+kr_panel_timing kr_gemm_take_timing(int groups, int waves);
 // Several products; on the small-M path those sharing M and K run in one
 // launch (independent outputs), otherwise they are launched in order.
 // Width (in 16-column panels) of the column groups the small-M fragment

@@ -853,23 +853,11 @@ int launch_panel(kr_gemm_multi mj, hipStream_t s) {
     }
     size_t lds = S > 1 ? (size_t)S * TM * NS * 256 * sizeof(float) : 0;
     if (QA && S > 1) lds += (size_t)S * TM * 16 * sizeof(float);
-    mj.stamps = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    if (t_panel_stamps) {
-        // the buffer holds KR_STAMP_WAVES slots for t_panel_cap workgroups
-        const bool fits = total <= t_panel_cap && S <= KR_STAMP_WAVES;
-        if (fits) {
-            mj.stamps = t_panel_stamps;
-            ev0 = t_panel_ev[0];
-            ev1 = t_panel_ev[1];
-        }
-        t_panel_stamps = nullptr;
-        t_panel_ev[0] = t_panel_ev[1] = nullptr;
-        t_panel_taken = fits ? total : -total;
-    }
-    if (ev0)
+    const kr_panel_timing tm = kr_gemm_take_timing(total, S);
+    mj.stamps = tm.stamps;
+    if (tm.start)
         hipExtLaunchKernelGGL(gemm_panel_kernel<TM, NS, FRAG, MAXT, I8, QA>, dim3(total),
-                              dim3(64 * S), (uint32_t)lds, s, ev0, ev1, 0u, mj);
+                              dim3(64 * S), (uint32_t)lds, s, tm.start, tm.stop, 0u, mj);
     else
         gemm_panel_kernel<TM, NS, FRAG, MAXT, I8, QA><<<total, dim3(64 * S), lds, s>>>(mj);
     KR_LAUNCHED();
@@ -888,6 +876,18 @@ void kr_gemm_time_next_panel(unsigned long long* stamps, int max_groups, hipEven
 }
 
 int kr_gemm_timed_launch_taken() { return t_panel_taken; }
+
+kr_panel_timing kr_gemm_take_timing(int groups, int waves) {
+    kr_panel_timing t{};
+    if (!t_panel_stamps) return t;
+    // the buffer holds KR_STAMP_WAVES slots for t_panel_cap workgroups
+    const bool fits = groups <= t_panel_cap && waves <= KR_STAMP_WAVES;
+    if (fits) t = kr_panel_timing{t_panel_stamps, t_panel_ev[0], t_panel_ev[1]};
+    t_panel_stamps = nullptr;
+    t_panel_ev[0] = t_panel_ev[1] = nullptr;
+    t_panel_taken = fits ? groups : -groups;
+    return t;
+}
 
 namespace {
 

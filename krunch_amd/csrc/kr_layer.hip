@@ -720,10 +720,9 @@ PrefetchSet att_stage_set(const kr_layer_weights& L, int C, int M, const Work& w
 // carried rows wait in the workspace's kx and fkx rows, which such a layer
 // does not use otherwise, until the next product copies them to the state.
 // Not for layer 0 of a forward from token ids, whose LN1-mix gathers the
-// embedding (or ran in the decode kernel), and not while that step's panel
-// products are timed (kr_step_timing's phases name separate launches).
-bool use_step_fused(int M, int F, bool i8, const EmbedSrc* e, const Phases& ph) {
-    return M <= (i8 ? KR_STEP_FUSE_M_I8 : KR_STEP_FUSE_M) && F % 256 == 0 && !e && !ph.stamps;
+// embedding (or ran in the decode kernel).
+bool use_step_fused(int M, int F, bool i8, const EmbedSrc* e) {
+    return M <= (i8 ? KR_STEP_FUSE_M_I8 : KR_STEP_FUSE_M) && F % 256 == 0 && !e;
 }
 
 kr_step_kvr step_kvr_args(const kr_layer_weights& L, const kr_half* x, int M, const kr_layer_state& st,
@@ -778,7 +777,7 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     const int M = B * T, G = C / 256;
     const bool fr = use_fragments_q8(Q, M);
     const bool mid = use_mid_q8(Q, M);      // fragment-packed, quantised by row kernels
-    if (fr && T == 1 && use_step_fused(M, F, true, e, ph)) {
+    if (fr && T == 1 && use_step_fused(M, F, true, e)) {
         KR_TRY(ph.mark(0));
         KR_TRY(ph.mark(1));
         KR_TRY(kr_step_launch_kvr(C, true, step_kvr_args(L, x, M, st, w), s));
@@ -891,7 +890,7 @@ int layer_step_fused(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
                      const kr_layer_state& st, const Work& w, hipStream_t s,
                      const EmbedSrc* e, const Phases& ph) {
     const int M = B, G = C / 256;
-    if (use_step_fused(M, F, false, e, ph)) {
+    if (use_step_fused(M, F, false, e)) {
         KR_TRY(ph.mark(0));
         KR_TRY(ph.mark(1));
         KR_TRY(kr_step_launch_kvr(C, false, step_kvr_args(L, x, M, st, w), s));
@@ -1103,8 +1102,8 @@ int profile_events() {
 // ---------------------------------------------------------------------------
 // Decode-step timing: when a phase p whose launch is a small-M panel product
 // is selected (3 output projection, 5 channel-mix R + K, 6 value product),
-// every layer of a stepped forward launches that product with a stamp
-// buffer: each of its waves stores its start and end on the 100 MHz steady
+// every layer of a stepped forward launches that product (5 in a layer of
+// four launches: with the LN2-mix that its launch holds) with a stamp buffer: each of its waves stores its start and end on the 100 MHz steady
 // counter (also inside a captured decode graph, at every replay). Outside
 // stream capture the launch also takes two HIP events through
 // hipExtLaunchKernel, which record its dispatch's start and end. Reading

@@ -38,6 +38,7 @@ struct kr_step_rk {
     kr_half* rf;               // [M, C] fp16(sigmoid(fp16(acc)))
     kr_half* kf;               // fragment-packed [M16, F] fp16(relu(fp16(acc))^2)
     int F, M;                  // F % 256 == 0
+    unsigned long long* stamps;   // decode-step timing (kr_gemm.h), set by the launch
 };
 
 int kr_step_launch_kvr(int C, bool i8, const kr_step_kvr& a, hipStream_t s);

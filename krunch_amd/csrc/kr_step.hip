@@ -22,6 +22,8 @@
 // B = 1 339 / 292, 8 355 / 329, 16 350 / 345, 40 369 / 340, 80 395 / 363,
 // 128 430 / 394, 160 465 / 453, 200 548 / 661; w8a8 B = 1 363 / 301,
 // 16 375 / 374, 40 393 / 377, 128 450 / 418, 144 447 / 466.
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -233,6 +235,7 @@ __global__ void __launch_bounds__(64 * S * P) ln_rk_kernel(kr_step_rk a) {
     __shared__ float sc[16];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const unsigned long long t_start = a.stamps ? (unsigned long long)wall_clock64() : 0ull;
     const int p = wave / S, s = wave % S;
     const int ng = (C + a.F) / (16 * NP);
     const int n_g = (int)blockIdx.x % ng, m0 = (int)blockIdx.x / ng * 16;
@@ -289,6 +292,11 @@ __global__ void __launch_bounds__(64 * S * P) ln_rk_kernel(kr_step_rk a) {
         if (isk) *reinterpret_cast<kr_half4*>(a.kf + kr_frag_index(m, n, a.F)) = y;
         else *reinterpret_cast<kr_half4*>(a.rf + (size_t)m * C + n) = y;
     }
+    if (a.stamps && lane == 0) {       // lane 0's row always exists
+        unsigned long long* st = a.stamps + 2 * (KR_STAMP_WAVES * blockIdx.x + wave);
+        st[0] = t_start;
+        st[1] = (unsigned long long)wall_clock64();
+    }
 }
 
 template <int S, bool I8>
@@ -297,6 +305,19 @@ int launch_kvr(const kr_step_kvr& a, hipStream_t s) {
     // one column panel per workgroup while that fits one round of the 256 CUs
     if (mt * ng <= 256) ln_kvr_wkv_kernel<S, 1, I8><<<mt * ng, 192 * S, 0, s>>>(a);
     else ln_kvr_wkv_kernel<S, 2, I8><<<mt * ng / 2, 192 * S, 0, s>>>(a);
+    KR_LAUNCHED();
+    return KR_OK;
+}
+
+template <int S, int P, int NS, bool I8>
+int launch_rk_shape(kr_step_rk a, int blocks, hipStream_t s) {
+    const kr_panel_timing tm = kr_gemm_take_timing(blocks, S * P);
+    a.stamps = tm.stamps;
+    if (tm.start)
+        hipExtLaunchKernelGGL((ln_rk_kernel<S, P, NS, I8>), dim3(blocks), dim3(64 * S * P), 0u, s,
+                              tm.start, tm.stop, 0u, a);
+    else
+        ln_rk_kernel<S, P, NS, I8><<<blocks, 64 * S * P, 0, s>>>(a);
     KR_LAUNCHED();
     return KR_OK;
 }
@@ -314,12 +335,10 @@ int launch_rk(const kr_step_rk& a, hipStream_t s) {
     int P = rows > 2 * held * S ? 4 : (rows > held * S ? 2 : 1);
     while (P < 4 && mt * panels / P > 256) P *= 2;
     const int blocks = mt * panels / P;
-    if (P == 1) ln_rk_kernel<S, 1, 1, I8><<<blocks, 64 * S, 0, s>>>(a);
-    else if (P == 2) ln_rk_kernel<S, 2, 1, I8><<<blocks, 128 * S, 0, s>>>(a);
-    else if (blocks <= 256) ln_rk_kernel<S, 4, 1, I8><<<blocks, 256 * S, 0, s>>>(a);
-    else ln_rk_kernel<S, 4, 2, I8><<<blocks / 2, 256 * S, 0, s>>>(a);
-    KR_LAUNCHED();
-    return KR_OK;
+    if (P == 1) return launch_rk_shape<S, 1, 1, I8>(a, blocks, s);
+    if (P == 2) return launch_rk_shape<S, 2, 1, I8>(a, blocks, s);
+    if (blocks <= 256) return launch_rk_shape<S, 4, 1, I8>(a, blocks, s);
+    return launch_rk_shape<S, 4, 2, I8>(a, blocks / 2, s);
 }
 
 }  // namespace

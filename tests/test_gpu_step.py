@@ -1,6 +1,8 @@
 """Stepped layers with the LN-mix inside the product launches (few streams)
 against packed windows over the same tokens, and the decode run's refusal of a
 stream under capture."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -55,3 +57,51 @@ def test_packed_product_refuses_more_than_512_rows():
     with pytest.raises(Exception, match="512"):
         _lib.call("kr_det_matmul_i8", xf.data_ptr(), out.data_ptr(), 513, 256, wf.data_ptr(),
                   out.data_ptr(), 256, out.data_ptr(), 256, 1, None, None, 1, _lib.stream_ptr())
+
+
+# layers of four launches and of six, both codecs
+@pytest.mark.parametrize("w8a8", [False, True])
+@pytest.mark.parametrize("B", [1, 5, 100, 200])
+def test_step_timing_leaves_the_launches_as_they_are(B, w8a8):
+    """A captured decode step has as many launches with a phase timed as
+    without; an eager one reports a dispatch and a wave span per layer."""
+    w = synthetic.make_weights(n_layer=3, V=1000, seed=B)
+    P = cpp_path.init_weights(w, "cuda", w8a8=w8a8)["prepared"]
+    dev = dict(device="cuda")
+    syms = torch.zeros(B, dtype=torch.int32, **dev)
+    bits = torch.zeros(64, dtype=torch.uint8, **dev)
+    ac = torch.zeros((B, 4), dtype=torch.uint32, **dev)
+    st = cpp_path.fresh_state_batched({"prepared": P}, B)
+    x = torch.zeros((B, P.C), dtype=torch.float16, **dev)
+    ws = torch.empty(_lib.lib().kr_forward_workspace_bytes(B, P.C, P.F), dtype=torch.uint8, **dev)
+    logits = torch.empty((B, P.V), dtype=torch.float16, **dev)
+    L = _lib.lib()
+    _lib.call("kr_decode_init_batched", bits.data_ptr(), 64, None, None, ac.data_ptr(), B, _lib.stream_ptr())
+
+    def step():
+        _lib.call("kr_decode_step", P.ptr, B, st.ptr, syms.data_ptr(), x.data_ptr(), ws.data_ptr(),
+                  ws.numel(), logits.data_ptr(), P.V, bits.data_ptr(), 64, None, None, ac.data_ptr(),
+                  None, 0, None, None, 24, _lib.stream_ptr())
+
+    def launches():
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            step()
+        n = ctypes.c_size_t(0)
+        assert L.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+        return n.value
+
+    try:
+        step()
+        plain = launches()
+        for phase in (3, 5, 6):
+            _lib.call("kr_step_timing", phase, None)
+            assert launches() == plain, phase
+            step()
+            us, span, n = (ctypes.c_double * 8)(), (ctypes.c_double * 8)(), ctypes.c_int(0)
+            _lib.call("kr_step_timing_read", us, span, 8, ctypes.byref(n))
+            assert n.value == 3
+            assert all(0.0 < us[i] < 1000.0 and 0.0 < span[i] < 1000.0 for i in range(3)), phase
+    finally:
+        L.kr_step_timing(-1, None)
+        cpp_path.release_weights(w)
