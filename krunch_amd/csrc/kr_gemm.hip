@@ -634,12 +634,16 @@ __global__ void __launch_bounds__(MAXT) gemm_panel_kernel(kr_gemm_multi mj) {
             }
         }
     }
-    // ---- row copy: this thread's first unit fetched here, stored at the end
+    // ---- row copy: this thread's first unit fetched here, stored at the end.
+    // Only in tiles of one row block, which panel_cost gives the launches with
+    // a copy: its four registers cost the 2 x 2 tile a wave per SIMD (the
+    // channel-mix R/K product at 176 rows 7.0 -> 8.2 us on MI355X).
+    constexpr bool COPY = FRAG && TM == 1;
     const int cp0 = bid * (int)blockDim.x + (int)threadIdx.x;
     uint2 cp_v;
-    if (FRAG && cp0 < mj.copy.n) cp_v = mj.copy.src[cp0];
+    if (COPY && cp0 < mj.copy.n) cp_v = mj.copy.src[cp0];
     auto copy_rows = [&]() {
-        if (!FRAG || cp0 >= mj.copy.n) return;
+        if (!COPY || cp0 >= mj.copy.n) return;
         mj.copy.dst[cp0] = cp_v;
         for (int u = cp0 + (int)(gridDim.x * blockDim.x); u < mj.copy.n; u += (int)(gridDim.x * blockDim.x))
             mj.copy.dst[u] = mj.copy.src[u];
@@ -925,7 +929,7 @@ long long panel_cost(const kr_gemm_multi& mj, PanelShape sh) {
     // (measured on MI355X at M = 256: the value product 7.4 us at TM 1 x NS 4
     // against 8.8 at 2 x 2, the output projection 5.2 against 5.9);
     // 4 panels only for int8 weights
-    if (mj.job[0].a_q16 && sh.TM > 1) return LLONG_MAX;
+    if ((mj.job[0].a_q16 || mj.copy.n > 0) && sh.TM > 1) return LLONG_MAX;
     if (!mj.job[0].i8 && sh.NS > 2 && !(sh.NS == 3 && sh.TM == 1)) return LLONG_MAX;
     // int8 operands: at most 2 row blocks (the stepped channel-mix R/K
     // product at M = 256: w8a8 decode 1,880 -> 1,919 KB/s at 2 x 2 against

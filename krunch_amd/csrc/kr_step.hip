@@ -223,9 +223,11 @@ __global__ void __launch_bounds__(192 * S) ln_kvr_wkv_kernel(kr_step_kvr a) {
 // ---------------------------------------------------------------------------
 // LN2-mix and the channel mix's R and K products: 16 rows x 16 P NS columns
 // of one of them per workgroup, wave (p, s) runs K slice s of the NS panels of
-// column part p.
+// column part p. TIMED (decode-step timing): waves store their start and end
+// times at a.stamps; kernels of their own, since the test of a pointer at the
+// start holds up the first loads (0.4 us per launch on MI355X).
 // ---------------------------------------------------------------------------
-template <int S, int P, int NS, bool I8>
+template <int S, int P, int NS, bool I8, bool TIMED>
 __global__ void __launch_bounds__(64 * S * P) ln_rk_kernel(kr_step_rk a) {
     constexpr int C = 256 * S, NW = S * P, RPW = (16 + NW - 1) / NW, QS = I8 ? 4 : 8;
     constexpr int KB = S * QS, NP = P * NS, TPW = (NP + NW - 1) / NW;
@@ -235,7 +237,7 @@ __global__ void __launch_bounds__(64 * S * P) ln_rk_kernel(kr_step_rk a) {
     __shared__ float sc[16];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const unsigned long long t_start = a.stamps ? (unsigned long long)wall_clock64() : 0ull;
+    const unsigned long long t_start = TIMED ? (unsigned long long)wall_clock64() : 0ull;
     const int p = wave / S, s = wave % S;
     const int ng = (C + a.F) / (16 * NP);
     const int n_g = (int)blockIdx.x % ng, m0 = (int)blockIdx.x / ng * 16;
@@ -292,7 +294,7 @@ __global__ void __launch_bounds__(64 * S * P) ln_rk_kernel(kr_step_rk a) {
         if (isk) *reinterpret_cast<kr_half4*>(a.kf + kr_frag_index(m, n, a.F)) = y;
         else *reinterpret_cast<kr_half4*>(a.rf + (size_t)m * C + n) = y;
     }
-    if (a.stamps && lane == 0) {       // lane 0's row always exists
+    if (TIMED && lane == 0) {          // lane 0's row always exists
         unsigned long long* st = a.stamps + 2 * (KR_STAMP_WAVES * blockIdx.x + wave);
         st[0] = t_start;
         st[1] = (unsigned long long)wall_clock64();
@@ -314,10 +316,12 @@ int launch_rk_shape(kr_step_rk a, int blocks, hipStream_t s) {
     const kr_panel_timing tm = kr_gemm_take_timing(blocks, S * P);
     a.stamps = tm.stamps;
     if (tm.start)
-        hipExtLaunchKernelGGL((ln_rk_kernel<S, P, NS, I8>), dim3(blocks), dim3(64 * S * P), 0u, s,
-                              tm.start, tm.stop, 0u, a);
+        hipExtLaunchKernelGGL((ln_rk_kernel<S, P, NS, I8, true>), dim3(blocks), dim3(64 * S * P), 0u,
+                              s, tm.start, tm.stop, 0u, a);
+    else if (tm.stamps)
+        ln_rk_kernel<S, P, NS, I8, true><<<blocks, 64 * S * P, 0, s>>>(a);
     else
-        ln_rk_kernel<S, P, NS, I8><<<blocks, 64 * S * P, 0, s>>>(a);
+        ln_rk_kernel<S, P, NS, I8, false><<<blocks, 64 * S * P, 0, s>>>(a);
     KR_LAUNCHED();
     return KR_OK;
 }
