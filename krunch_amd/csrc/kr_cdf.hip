@@ -44,7 +44,7 @@ constexpr int kMaxLevels = 16;               // tree height above the leaves
 constexpr int kMaxBlocks = 8;                // 8192-element blocks: V <= 65536
 
 enum : int { IN_LOGITS_F16 = 0, IN_PROBS_F32 = 1 };
-enum : int { M_CDF = 0, M_COUNTS = 1, M_PROBS = 2, M_PAIRS = 3, M_DECODE = 4 };
+enum : int { M_CDF = 0, M_COUNTS = 1, M_PROBS = 2, M_PAIRS = 3, M_DECODE = 4, M_CDF_SPAN = 5 };
 
 struct PlanArgs {
     const int2* leaves;      // (start, len), index order
@@ -177,79 +177,82 @@ __device__ __forceinline__ StageMap stage_row(const kr_half* __restrict__ rp, in
 }
 
 // ---------------------------------------------------------------------------
-// Whole CDF (or count) rows leave through LDS. A thread holds counts of
-// scattered leaves, 8 consecutive elements per 8-lane group, and a row of
-// int32 starts at any 4-byte address, so stores from that layout write 32-byte
-// pieces and a scan over them in memory reads lanes 200 bytes apart. Instead
-// the counts of up to 32768 elements at a time (4 blocks of the summation, so
-// no leaf is split) go into the stage, which the gathered row has left; every
-// thread scans one run of kSpanRun elements there, and the results are stored
-// with consecutive lanes on consecutive words. Element i of a span sits at
-// word i + 4 (i / 32): the 16-byte reads of 16 neighbouring runs (36 words
-// apart) then hit all banks once.
+// Whole CDF rows of kSpanMinV elements and more leave through LDS
+// (M_CDF_SPAN). A thread holds counts of scattered leaves, 8 consecutive
+// elements per 8-lane group, and a row of int32 starts at any 4-byte address,
+// so stores from that layout (M_CDF, M_COUNTS) write 32-byte pieces and a scan
+// over them in memory reads lanes 200 bytes apart. Instead the counts of up to
+// 32768 elements at a time (4 blocks of the summation, so no leaf is split) go
+// into the stage, which the gathered row has left; every thread scans one run
+// of kSpanRun elements there, and the results are stored with consecutive
+// lanes on consecutive words. Element i of a span sits at word i + 4 (i / 32):
+// the 16-byte reads of 16 neighbouring runs (36 words apart) then hit all
+// banks once.
 // Bound: the row's own VALU phases (about 20 us per row and CU). Measured on
-// MI355X, 300 rows x 50277: 447 us from the leaf layout, 79 us through LDS (256
-// rows, one per CU: 45 us, of which 13 us are the output).
+// MI355X, from the leaf layout / through LDS, us: 300 rows x 50277 449 / 78
+// (256 rows, one per CU: 366 / 43), 256 rows x 8192 21.6 / 16.5, x 6000
+// 16.1 / 16.4, x 4096 13.5 / 15.2, x 1000 10.6 / 14.0 (a run per thread is
+// serial however short the row is, so short rows keep the leaf layout). Count
+// rows need no scan and keep it at any length: 256 rows x 50277 34.0 / 36.6,
+// one row 18.7 / 26.4.
 // ---------------------------------------------------------------------------
+constexpr int kSpanMinV = 8192;
 constexpr int kSpan = 32768;
 constexpr int kSpanRun = kSpan / kThreads;
 constexpr int kSpanWords = kSpan + kSpan / 8;
 __device__ __forceinline__ int span_pos(int i) { return i + ((i >> 5) << 2); }
 
-// Scan (SCAN) or leave as they are n counts in `cnt`, add `carry`, and store
-// them at orow[0 .. n). Returns the last inclusive sum. Every thread calls it;
-// the counts were written by the callers' threads before.
-template <bool SCAN>
+// Scan n counts in `cnt` from `carry` and store the sums at orow[0 .. n).
+// Returns the last inclusive sum. Every thread calls it; the counts were
+// written by the callers' threads before.
 __device__ __forceinline__ int span_out(int* cnt, int n, int carry, int32_t* __restrict__ orow,
                                         int* redi, int tid, int lane, int wave) {
     static_assert(kSpanRun == 32, "a run is one skew segment");
     __syncthreads();
-    if constexpr (SCAN) {
-        // two passes over the run in LDS (its sum, then its prefix sums): the
-        // q values still held leave no registers for 32 counts
-        const int i0 = tid * kSpanRun;
-        int4* run = reinterpret_cast<int4*>(cnt + span_pos(i0));
-        auto quad = [&](int q) {                 // words past n hold no count
-            int4 w = run[q];
-            const int i = i0 + 4 * q;
-            w.x = i < n ? w.x : 0;
-            w.y = i + 1 < n ? w.y : 0;
-            w.z = i + 2 < n ? w.z : 0;
-            w.w = i + 3 < n ? w.w : 0;
-            return w;
-        };
-        int local = 0;
-        #pragma unroll 4
-        for (int q = 0; q < kSpanRun / 4; q++) {
-            const int4 w = quad(q);
-            local += (w.x + w.y) + (w.z + w.w);
-        }
-        int incl = local;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int up = __shfl_up(incl, o);
-            if (lane >= o) incl += up;
-        }
-        if (lane == 63) redi[wave] = incl;
-        __syncthreads();
-        int base = carry + incl - local;
-        int all = carry;
-        for (int w = 0; w < kWaves; w++) {
-            if (w < wave) base += redi[w];
-            all += redi[w];
-        }
-        #pragma unroll 4
-        for (int q = 0; q < kSpanRun / 4; q++) {
-            int4 w = quad(q);
-            w.x += base;
-            w.y += w.x;
-            w.z += w.y;
-            w.w += w.z;
-            base = w.w;
-            run[q] = w;
-        }
-        carry = all;
-        __syncthreads();
+    // two passes over the run in LDS (its sum, then its prefix sums): the
+    // q values still held leave no registers for 32 counts
+    const int i0 = tid * kSpanRun;
+    int4* run = reinterpret_cast<int4*>(cnt + span_pos(i0));
+    auto quad = [&](int q) {                     // words past n hold no count
+        int4 w = run[q];
+        const int i = i0 + 4 * q;
+        w.x = i < n ? w.x : 0;
+        w.y = i + 1 < n ? w.y : 0;
+        w.z = i + 2 < n ? w.z : 0;
+        w.w = i + 3 < n ? w.w : 0;
+        return w;
+    };
+    int local = 0;
+    #pragma unroll 4
+    for (int q = 0; q < kSpanRun / 4; q++) {
+        const int4 w = quad(q);
+        local += (w.x + w.y) + (w.z + w.w);
     }
+    int incl = local;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int up = __shfl_up(incl, o);
+        if (lane >= o) incl += up;
+    }
+    if (lane == 63) redi[wave] = incl;
+    __syncthreads();
+    int base = carry + incl - local;
+    int all = carry;
+    for (int w = 0; w < kWaves; w++) {
+        if (w < wave) base += redi[w];
+        all += redi[w];
+    }
+    #pragma unroll 4
+    for (int q = 0; q < kSpanRun / 4; q++) {
+        int4 w = quad(q);
+        w.x += base;
+        w.y += w.x;
+        w.z += w.y;
+        w.w += w.z;
+        base = w.w;
+        run[q] = w;
+    }
+    carry = all;
+    __syncthreads();
     // eight words per thread read before they are stored
     for (int i0 = tid; i0 < n; i0 += 8 * kThreads) {
         int c[8];
@@ -624,7 +627,7 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
     int lsum[kMaxIt];
     int bslot = -1;                       // 32 * it + k of the first maximum held
     int32_t* orow = nullptr;
-    if constexpr (MODE == M_CDF || MODE == M_COUNTS)
+    if constexpr (MODE == M_CDF || MODE == M_COUNTS || MODE == M_CDF_SPAN)
         orow = reinterpret_cast<int32_t*>(out) + (size_t)row * (size_t)out_ld;
     // A lane only notes, per register slice, whether any of its slots holds
     // p == pmax (one compare per element, the flags kept as lane masks); the
@@ -652,6 +655,10 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
             const float p = div_by(v[it][k], denom, rdenom);
             const int f = scaled_floor<IN>(p, scale);
             ls += f;
+            if constexpr (MODE == M_CDF || MODE == M_COUNTS) {
+                const bool live = k < 16 ? (k < nf) : (j < rm);
+                if (live) orow[slot_index(start[it], len[it], j, k) + 1] = f + 1;
+            }
             any_hit[it] = any_hit[it] || is_hit(it, k, p);
         }
         lsum[it] = ls + nf + (j < rm ? 1 : 0);
@@ -739,7 +746,8 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
         sh.amax = gi;
         sh.deficit = deficit;
         sh.amax_leaf = gL;
-        if constexpr (MODE == M_CDF || MODE == M_COUNTS) orow[0] = 0;
+        if constexpr (MODE == M_CDF || MODE == M_COUNTS) orow[gi + 1] += deficit;
+        if constexpr (MODE == M_CDF || MODE == M_COUNTS || MODE == M_CDF_SPAN) orow[0] = 0;
         if constexpr (MODE == M_PAIRS) {
             int pre = 0, cs = 0;
             for (int w = 0; w < kWaves; w++) { pre += sh.redi3[w]; cs += sh.redL[w]; }
@@ -749,9 +757,32 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
         }
         if constexpr (MODE == M_DECODE) sh.leaf_count[gL] += deficit;
     }
-    if constexpr (MODE == M_PAIRS) return;
+    if constexpr (MODE == M_PAIRS || MODE == M_COUNTS) return;
 
-    if constexpr (MODE == M_CDF || MODE == M_COUNTS) {
+    if constexpr (MODE == M_CDF) {
+        // Inclusive scan of counts over contiguous per-thread segments.
+        __syncthreads();
+        const int seg = (V + kThreads - 1) / kThreads;
+        const int i0 = min(V, tid * seg), i1 = min(V, i0 + seg);
+        int local = 0;
+        for (int i = i0; i < i1; i++) local += orow[i + 1];
+        int incl = local;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(incl, o);
+            if (lane >= o) incl += up;
+        }
+        if (lane == 63) sh.redi[wave] = incl;
+        __syncthreads();
+        int base = incl - local;
+        for (int w = 0; w < wave; w++) base += sh.redi[w];
+        for (int i = i0; i < i1; i++) {
+            base += orow[i + 1];
+            orow[i + 1] = base;
+        }
+        return;
+    }
+
+    if constexpr (MODE == M_CDF_SPAN) {
         __syncthreads();
         const int gi = sh.amax, deficit = sh.deficit;
         int* cnt = reinterpret_cast<int*>(stage);
@@ -782,8 +813,7 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
                 __syncthreads();
                 if (tid == 0) cnt[span_pos(gi - s0)] += deficit;
             }
-            carry = span_out<MODE == M_CDF>(cnt, min(kSpan, V - s0), carry, orow + s0 + 1, sh.redi,
-                                            tid, lane, wave);
+            carry = span_out(cnt, min(kSpan, V - s0), carry, orow + s0 + 1, sh.redi, tid, lane, wave);
         }
         return;
     }
@@ -899,11 +929,11 @@ __device__ __forceinline__ void cdf_row(const void* __restrict__ input, long lon
 
 // Halves of stage a kernel needs: the staged fp16 row, or the counts of a span.
 template <int IN, int MODE>
-constexpr int kStageUsed = MODE == M_CDF || MODE == M_COUNTS ? 2 * kSpanWords
-                           : IN == IN_LOGITS_F16            ? kStageMax
-                                                            : 8;
+constexpr int kStageUsed = MODE == M_CDF_SPAN ? 2 * kSpanWords
+                           : IN == IN_LOGITS_F16 ? kStageMax
+                                                 : 8;
 static_assert(2 * kSpanWords >= kStageMax && 4 * kSpanWords + sizeof(RowShared) <= 160 * 1024,
-              "the stage of a full-row kernel holds a row or a span of counts, in a CU's LDS");
+              "the stage of a spanned kernel holds a row or a span of counts, in a CU's LDS");
 
 template <int IN, int MODE>
 __global__ void __launch_bounds__(kThreads)
@@ -1125,6 +1155,14 @@ int launch_rows(const void* in, long long ld, int N, int V, int prec, void* out,
     return KR_OK;
 }
 
+// Cumulative rows [N, V + 1]; the line between the two ways out: kSpanMinV.
+template <int IN>
+int launch_cdf_rows(const void* in, long long ld, int N, int V, int prec, void* out, void* stream) {
+    if (V >= kSpanMinV)
+        return launch_rows<IN, M_CDF_SPAN>(in, ld, N, V, prec, out, V + 1, nullptr, DecodeArgs{}, stream);
+    return launch_rows<IN, M_CDF>(in, ld, N, V, prec, out, V + 1, nullptr, DecodeArgs{}, stream);
+}
+
 }  // namespace
 
 // kr_softmax_cdf_decode, plus (em non-null) layer 0's LN1-mix of each decoded
@@ -1161,8 +1199,7 @@ int kr_probs_to_cdf(const float* probs, int N, int V, long long ld, uint32_t* cd
                     int cdf_precision, void* stream) {
     KR_REQUIRE(probs && cdf_out, "kr_probs_to_cdf: null pointer");
     KR_REQUIRE(ld >= V, "kr_probs_to_cdf: ld %lld < V %d", ld, V);
-    return launch_rows<IN_PROBS_F32, M_CDF>(probs, ld, N, V, cdf_precision, cdf_out, V + 1,
-                                            nullptr, DecodeArgs{}, stream);
+    return launch_cdf_rows<IN_PROBS_F32>(probs, ld, N, V, cdf_precision, cdf_out, stream);
 }
 
 int kr_softmax_cdf(const uint16_t* logits, int N, int V, long long ld, int32_t* out,
@@ -1170,8 +1207,7 @@ int kr_softmax_cdf(const uint16_t* logits, int N, int V, long long ld, int32_t* 
     KR_REQUIRE(logits && out, "kr_softmax_cdf: null pointer");
     KR_REQUIRE(ld >= V, "kr_softmax_cdf: ld %lld < V %d", ld, V);
     if (cumulative)
-        return launch_rows<IN_LOGITS_F16, M_CDF>(logits, ld, N, V, cdf_precision, out, V + 1,
-                                                 nullptr, DecodeArgs{}, stream);
+        return launch_cdf_rows<IN_LOGITS_F16>(logits, ld, N, V, cdf_precision, out, stream);
     return launch_rows<IN_LOGITS_F16, M_COUNTS>(logits, ld, N, V, cdf_precision, out, V + 1,
                                                 nullptr, DecodeArgs{}, stream);
 }

@@ -166,3 +166,20 @@ def test_full_rows_at_span_edges(V):
     np.testing.assert_array_equal(counts[:, 1:], np.diff(ref.astype(np.int64), axis=1))
     q = osm.softmax_probs(lg)
     np.testing.assert_array_equal(krunch_ac.probs_to_cdf(q), ref)
+
+
+@pytest.mark.parametrize("V", [31, 4096, 8191, 8192, 8193, 9000])
+def test_rows_on_both_sides_of_the_span_line(V):
+    """CDF rows from logits and from probabilities, and count rows, where
+    rows change from the leaf layout to spans in LDS."""
+    lg = _logits(5, V, V)
+    lg[0, :] = 1.5                          # all equal
+    lg[1, V - 1] = 40.0                     # the maximum, and its deficit, in the last element
+    ref = osm.logits_to_cdf(lg)
+    d = torch.from_numpy(lg).to(DEV)
+    np.testing.assert_array_equal(ops.softmax_cdf(d).cpu().numpy().view(np.uint32), ref)
+    counts = ops.det_softmax_cdf(d, 1 << 24).cpu().numpy()
+    assert (counts[:, 0] == 0).all()
+    np.testing.assert_array_equal(counts[:, 1:], np.diff(ref.astype(np.int64), axis=1))
+    p = osm.softmax_probs(lg)
+    np.testing.assert_array_equal(krunch_ac.probs_to_cdf(p), ocdf.probs_to_cdf(p))
