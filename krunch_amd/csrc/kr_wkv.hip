@@ -284,9 +284,13 @@ int kr_wkv_launch(const kr_wkv_args& a, bool det, hipStream_t s) {
     // division make the chain longer, scan ahead by 146 us per layer at
     // B = 32, by 42 at B = 48, behind by 24 at B = 64. Below 32 tokens
     // (one chunk) its five stages cost more than they hide: B = 64, T = 16
-    // 9 / 16 us.
+    // 9 / 16 us. At one to two chunks the pipeline's fill is a good part of
+    // the run, so the crossover comes earlier: fp16 T = 33, B = 16 / 24 / 32
+    // 8.7 / 8.8 / 8.8 (wkv_kernel) against 7.4 / 9.8 / 10.7; w8a8 T = 40, a
+    // layer at B = 44 3 us ahead, at B = 53 3 us behind.
     const long long wgs = (long long)a.B * ((a.C + kScanCh - 1) / kScanCh);
-    const bool scan = a.T >= 32 && wgs <= (det ? 2560 : 1536);
+    const long long most = a.T < 64 ? (det ? 2048 : 1024) : (det ? 2560 : 1536);
+    const bool scan = a.T >= 32 && wgs <= most;
     if (scan) {
         const dim3 grid((a.C + kScanCh - 1) / kScanCh, a.B);
         if (det) wkv_scan_kernel<true><<<grid, kScanThreads, 0, s>>>(a);

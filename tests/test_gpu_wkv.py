@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from krunch_amd import _lib
+from krunch_amd import _lib, cpp_path, synthetic
 from oracle import rwkv4
 
 pytestmark = pytest.mark.gpu
@@ -46,3 +46,25 @@ def test_packed_wkv_equals_token_by_token(B, T, C):
     # of exp and reciprocal errors far below that
     ref = (r.float().cpu() * y).numpy()
     np.testing.assert_allclose(got.float().cpu().numpy(), ref, rtol=2.0 ** -9, atol=2.0 ** -9)
+
+
+# the last workgroup count that takes the time-split kernel and the first that
+# does not, at one to two chunks and above, per codec; T short of and past a chunk
+@pytest.mark.parametrize("w8a8,B,T", [(False, 64, 33), (False, 65, 33), (False, 96, 65), (False, 97, 65),
+                                      (True, 128, 40), (True, 129, 40), (True, 160, 64), (True, 161, 64)])
+def test_layers_on_both_sides_of_the_split_line(w8a8, B, T):
+    """Packed layers whose WKV changes kernels against the same tokens one
+    stream at a time (always the time-split kernel): equal bit for bit."""
+    w = synthetic.make_weights(n_layer=2, C=256, F=512, V=300, seed=3)
+    W = cpp_path.init_weights(w, "cuda", w8a8=w8a8)
+    try:
+        ids = torch.from_numpy(synthetic.zipf_tokens(B, T, V=300))
+        st = cpp_path.fresh_state_batched(W, B)
+        got = cpp_path.forward_packed_batched(W, ids, st).view(B, T, -1)
+        for b in (0, B // 2, B - 1):
+            st1 = cpp_path.fresh_state_batched(W, 1)
+            assert torch.equal(cpp_path.forward_packed_batched(W, ids[b:b + 1], st1), got[b]), b
+            for x, y in zip(st1.flat(), st.flat()):
+                assert torch.equal(x[0], y[b]), b
+    finally:
+        cpp_path.release_weights(w)
