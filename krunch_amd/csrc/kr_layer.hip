@@ -721,8 +721,8 @@ PrefetchSet att_stage_set(const kr_layer_weights& L, int C, int M, const Work& w
 // does not use otherwise, until the next product copies them to the state.
 // Not for layer 0 of a forward from token ids, whose LN1-mix gathers the
 // embedding (or ran in the decode kernel).
-bool use_step_fused(int M, int F, bool i8, const EmbedSrc* e) {
-    return M <= (i8 ? KR_STEP_FUSE_M_I8 : KR_STEP_FUSE_M) && F % 256 == 0 && !e;
+bool use_step_fused(int C, int M, int F, bool i8, const EmbedSrc* e) {
+    return kr_step_fuse_ok(C, M, i8) && F % 256 == 0 && !e;
 }
 
 kr_step_kvr step_kvr_args(const kr_layer_weights& L, const kr_half* x, int M, const kr_layer_state& st,
@@ -777,7 +777,7 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     const int M = B * T, G = C / 256;
     const bool fr = use_fragments_q8(Q, M);
     const bool mid = use_mid_q8(Q, M);      // fragment-packed, quantised by row kernels
-    if (fr && T == 1 && use_step_fused(M, F, true, e)) {
+    if (fr && T == 1 && use_step_fused(C, M, F, true, e)) {
         KR_TRY(ph.mark(0));
         KR_TRY(ph.mark(1));
         KR_TRY(kr_step_launch_kvr(C, true, step_kvr_args(L, x, M, st, w), s));
@@ -890,7 +890,7 @@ int layer_step_fused(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
                      const kr_layer_state& st, const Work& w, hipStream_t s,
                      const EmbedSrc* e, const Phases& ph) {
     const int M = B, G = C / 256;
-    if (use_step_fused(M, F, false, e)) {
+    if (use_step_fused(C, M, F, false, e)) {
         KR_TRY(ph.mark(0));
         KR_TRY(ph.mark(1));
         KR_TRY(kr_step_launch_kvr(C, false, step_kvr_args(L, x, M, st, w), s));

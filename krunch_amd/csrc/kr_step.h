@@ -2,10 +2,23 @@
 #pragma once
 #include "kr_gemm.h"
 
-// Streams up to which they are used: beyond, the LN that every column group
-// repeats costs more than the launches it saves (figures in kr_step.hip).
-#define KR_STEP_FUSE_M 160
-#define KR_STEP_FUSE_M_I8 128
+// Whether a stepped layer of M streams takes them: beyond, the LN that every
+// column group repeats (C / 16 groups of C values per row) costs more than the
+// launches it saves. Measured on MI355X, one step of 12 layers, F = 4 C, us,
+// six launches per layer / four. fp16: C = 256, M = 16 210 / 196, 160 274 / 223;
+// 512, 16 266 / 235, 160 344 / 275; 768, 16 292 / 272, 128 370 / 324, 144
+// 373 / 374, 160 376 / 379; 1024, 8 332 / 316, 48 352 / 347, 64 379 / 384, 96
+// 408 / 434, 128 437 / 517. w8a8, whose rows are quantised as well: C = 256, 12
+// 240 / 231, 16 240 / 261, 96 263 / 269, 97 301 / 271 (the panel products'
+// tiles change there), 128 304 / 278; 512, 16 302 / 288, 128 354 / 311; 768, 16
+// 327 / 325, 128 399 / 361; 1024, 16 362 / 350, 96 421 / 389, 112 435 / 453.
+// (decode runs of 136..160 streams, C = 768, fp16: 1-2 % faster with six). The
+// limits at C <= 512 (fp16) and 512..768 (w8a8) are the last rows measured
+// ahead, not crossovers.
+inline bool kr_step_fuse_ok(int C, int M, bool i8) {
+    if (i8) return C <= 256 ? M <= 12 || (M > 96 && M <= 128) : M <= (C <= 768 ? 128 : 96);
+    return M <= (C <= 512 ? 160 : (C <= 768 ? 128 : 48));
+}
 
 struct kr_step_ln {
     const kr_half* x;          // [M, C] residual stream

@@ -1,5 +1,5 @@
 // Stepped (T = 1) layer products with the LayerNorm-mix that feeds them in
-// the same launch, for up to KR_STEP_FUSE_M streams. The decode step at these
+// the same launch, for few streams (kr_step_fuse_ok). The decode step at these
 // sizes is a chain of dependent launches, each a memory round trip and a
 // dispatch, and these two kernels take two of a layer's six away.
 //

@@ -105,3 +105,12 @@ def test_step_timing_leaves_the_launches_as_they_are(B, w8a8):
     finally:
         L.kr_step_timing(-1, None)
         cpp_path.release_weights(w)
+
+
+# the last row counts of four launches per layer and the first of six, at the
+# widths and codecs whose lines are not among the sizes above
+@pytest.mark.parametrize("C,w8a8,Bs", [(256, False, (160, 161)), (256, True, (12, 13, 96, 97, 128, 129)),
+                                       (512, True, (128, 129)), (1024, False, (48, 49)),
+                                       (1024, True, (96, 97))])
+def test_stepped_equals_packed_at_the_lines(C, w8a8, Bs):
+    test_stepped_equals_packed(C, Bs, w8a8)
