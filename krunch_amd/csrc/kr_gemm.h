@@ -84,14 +84,24 @@ __host__ __device__ inline long long kr_frag_rows(long long R) { return (R + 15)
 // which also reads and writes fragment-packed operands.
 #define KR_GEMM_SMALL_M 512
 #define KR_GEMM_SMALL_MAX_N 16384
-// Fragment-packed products of more rows than that, up to this many, take the
-// register-fed kernel of kr_mid.hip. Measured on MI355X (one layer, us, tile
-// kernel / register-fed): fp16 157.6 / 155.7 at 2200 rows, 163.6 / 163.3 at
-// 2400, 178.7 / 194.5 at 2700; w8a8, with half the operand bytes, 119.3 /
-// 115.5 at 1500, 126.1 / 127.8 at 1800 (kr_layer.hip asks for fragment-packed
-// operands up to these limits).
+// Fragment-packed products of more rows than that, up to this many (the int8
+// limit apart), take the register-fed kernel of kr_mid.hip.
 #define KR_GEMM_MID_M 2304
 #define KR_GEMM_MID_M_I8 1664
+// Rows up to which a layer of width C asks for fragment-packed operands, and
+// so for that kernel; more rows are row-major in the tile kernels. Measured on
+// MI355X, us, tile kernels / register-fed, a layer called again and again (its
+// weights in L2) and 12 layers in turn: fp16 C = 512, 2304 rows 124 / 118 and
+// 1337 / 1236; 768, 2176 rows 156 / 155 and 1949 / 1800, 2304 157 / 165 and
+// 1939 / 1873; 1024, 1856 rows 187 / 186 and 2526 / 2175, 2048 189 / 201 and
+// 2606 / 2514, 2112 219 / 233 and 2712 / 2882. w8a8, with half the operand
+// bytes: 512, 1664 rows 111 / 96 and 1223 / 1028; 768, 1664 rows 135 / 131 and
+// 1510 / 1463; 1024, 1536 rows 161 / 159 and 1912 / 1783, 1664 162 / 169 and
+// 1941 / 1908.
+inline int kr_gemm_mid_rows(int C, bool i8) {
+    if (i8) return C <= 768 ? KR_GEMM_MID_M_I8 : 1536;
+    return C <= 512 ? KR_GEMM_MID_M : (C <= 768 ? 2176 : 1856);
+}
 
 // A row copy that rides along in a small-M product launch (8-byte units,
 // 8-byte aligned): the carried rows a fused LN-mix left beside the state it

@@ -570,16 +570,15 @@ bool use_fragments_q8(const kr_layer_q8& Q, long long M) {
            Q.fR.qf;
 }
 
-// Above that, up to KR_GEMM_MID_M rows (w8a8 KR_GEMM_MID_M_I8), the products
-// read fragment-packed operands as well, in the register-fed kernel of
-// kr_mid.hip.
-bool use_mid(const kr_layer_weights& L, long long M) {
-    return M > KR_GEMM_SMALL_M && M <= KR_GEMM_MID_M && L.Kf && L.Vf && L.Rf && L.Of && L.fKf &&
-           L.fVf && L.fRf;
+// Above that, up to kr_gemm_mid_rows, the products read fragment-packed
+// operands as well, in the register-fed kernel of kr_mid.hip.
+bool use_mid(const kr_layer_weights& L, int C, long long M) {
+    return M > KR_GEMM_SMALL_M && M <= kr_gemm_mid_rows(C, false) && L.Kf && L.Vf && L.Rf && L.Of &&
+           L.fKf && L.fVf && L.fRf;
 }
-bool use_mid_q8(const kr_layer_q8& Q, long long M) {
-    return M > KR_GEMM_SMALL_M && M <= KR_GEMM_MID_M_I8 && Q.K.qf && Q.V.qf && Q.R.qf && Q.O.qf &&
-           Q.fK.qf && Q.fV.qf && Q.fR.qf;
+bool use_mid_q8(const kr_layer_q8& Q, int C, long long M) {
+    return M > KR_GEMM_SMALL_M && M <= kr_gemm_mid_rows(C, true) && Q.K.qf && Q.V.qf && Q.R.qf &&
+           Q.O.qf && Q.fK.qf && Q.fV.qf && Q.fR.qf;
 }
 
 // Layer 0's LN1-mix can run in the previous decode kernel (kr_embed_mix)
@@ -776,7 +775,7 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
     const kr_layer_q8& Q = *L.q8;
     const int M = B * T, G = C / 256;
     const bool fr = use_fragments_q8(Q, M);
-    const bool mid = use_mid_q8(Q, M);      // fragment-packed, quantised by row kernels
+    const bool mid = use_mid_q8(Q, C, M);      // fragment-packed, quantised by row kernels
     if (fr && T == 1 && use_step_fused(C, M, F, true, e)) {
         KR_TRY(ph.mark(0));
         KR_TRY(ph.mark(1));
@@ -978,7 +977,7 @@ int layer_forward(const kr_layer_weights& L, int C, int F, kr_half* x, int B, in
                "fragment-packed weights (fp16 or w8a8)");
     if (L.q8) return layer_forward_q8(L, C, F, x, B, T, st, w, s, e, ph);
     const int M = B * T, G = C / 256;
-    const bool fr = use_fragments(L, M) || use_mid(L, M);
+    const bool fr = use_fragments(L, M) || use_mid(L, C, M);
     if (use_fragments(L, M) && T == 1) return layer_step_fused(L, C, F, x, B, st, w, s, e, ph);
     LnMixArgs a{};
     a.x = x;

@@ -85,3 +85,24 @@ def test_head_rows_equals_single_blocks(C, V, M, ld):
         assert bool((got[:, V:] == 7.0).all())
     finally:
         cpp_path.release_weights(w)
+
+
+# the last row counts of the register-fed kernel and the first past it, where
+# the line lies elsewhere than above
+@pytest.mark.parametrize("C,w8a8,B,T", [(768, False, 17, 128), (768, False, 7, 311), (1024, False, 1, 1856),
+                                        (1024, False, 3, 619), (1024, True, 3, 512), (1024, True, 29, 53),
+                                        (256, False, 9, 256), (256, False, 5, 461)])
+def test_windows_on_both_sides_of_the_lines(C, w8a8, B, T):
+    w = synthetic.make_weights(n_layer=2, C=C, F=4 * C, V=500, seed=C)
+    W = cpp_path.init_weights(w, "cuda", w8a8=w8a8)
+    try:
+        ids = torch.from_numpy(synthetic.zipf_tokens(B, T, V=500, seed_base=B + T))
+        st, st2 = (cpp_path.fresh_state_batched(W, B) for _ in range(2))
+        whole = cpp_path.forward_packed_batched(W, ids, st).view(B, T, -1)
+        step = 512 // B
+        parts = [cpp_path.forward_packed_batched(W, ids[:, i:i + step].contiguous(), st2).view(
+            B, -1, whole.shape[-1]) for i in range(0, T, step)]
+        assert torch.equal(whole, torch.cat(parts, 1))
+        assert torch.equal(st.buf, st2.buf)
+    finally:
+        cpp_path.release_weights(w)
