@@ -185,8 +185,10 @@ int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* epilogues, int njo
 bool kr_gemm_head_small_ok(int M, int N, int K);
 int kr_gemm_head_small(const kr_half* Af, const kr_half* Wf, int M, int N, int K, kr_half* out,
                        long long ldo, hipStream_t stream);
-// The same for M > 512 (kr_head.hip): any ldo >= N below 2^24.
-bool kr_gemm_head_rows_ok(int M, int N, int K);
+// The same for M > 512 (kr_head.hip): any ldo >= N below 2^24. _ok: it takes
+// these sizes; _faster: and it is the faster one, against kr_gemm_head_big.
+bool kr_gemm_head_rows_ok(int M, int N, int K, long long ldo);
+bool kr_gemm_head_rows_faster(int M, int N, int K, const kr_half* out, long long ldo);
 int kr_gemm_head_rows(const kr_half* Af, const kr_half* Wf, int M, int N, int K, kr_half* out,
                       long long ldo, hipStream_t stream);
 // The same product for any M: A [M, K] row-major (row stride lda), W^T [N, K]

@@ -2,6 +2,7 @@
 // step's kernel takes: 256 rows per workgroup held in registers, the weights
 // streamed past them. A file of its own: kernels added to kr_gemm.hip move the
 // decode step's panel kernels.
+#include <algorithm>
 #include <type_traits>
 
 #include "kr_gemm.h"
@@ -202,24 +203,68 @@ __global__ void __launch_bounds__(256, 1) gemm_head_rows_kernel(
 
 }  // namespace
 
-bool kr_gemm_head_rows_ok(int M, int N, int K) {
-    return M > 512 && N >= 1 && (K == 256 || K == 512 || K == 768);
+namespace {
+
+// one workgroup per CU: as many column runs (whole eights) as the row groups
+// leave; more than 32 row groups go in several launches
+constexpr int kLaunchRows = 32 * 256;
+
+int column_runs(int row_groups, int N) {
+    const int nb = (N + 15) / 16, most = 256 / row_groups;
+    const int n = nb < most ? nb : most;
+    return n >= 8 ? n & ~7 : n;
+}
+
+}  // namespace
+
+bool kr_gemm_head_rows_ok(int M, int N, int K, long long ldo) {
+    return M > 512 && N >= 1 && (K == 256 || K == 512 || K == 768) && ldo >= N && ldo < (1ll << 24);
+}
+
+// Where the 256 x 256 kernel stores 2 bytes at a time this one is faster, but
+// for few columns over several launches (V = 1000, odd stride, K = 768, 12288
+// rows 1.09 of its time). Where it stores 8 (stride and start multiples of
+// them), measured on MI355X as this kernel's time over its:
+//  * strides of whole 4096 bytes put the 16 rows of a store instruction on one
+//    memory channel: V = 65536, M = 1024 0.84..0.89, 1280 0.87..1.47, 2048
+//    1.7..2.6, 8192 1.9..2.2;
+//  * few columns share the load of the rows among few blocks: V = 1000, M =
+//    4096 0.80, 8192 1.02..1.08, 16384 1.4..1.6;
+//  * K = 256 and 512, whose rows hold fewer MFMAs per output: once the output
+//    outgrows the memory-side cache its partial lines cost memory time (V =
+//    50277, K = 256, M = 2048 0.74, 3072 1.43; K = 512, 2048 0.86..1.02, 4096
+//    1.11); K = 768 hides that (8192 0.90);
+//  * the longest column run against the rounds of 256 x 256 tiles, each about
+//    21.5 blocks of 16 columns long, the load of the rows 8: K = 768, V = 50277,
+//    M = 1280 (74 blocks, 4 rounds) 0.88, 6144 (401, 19) 0.96, 2816 (205, 9) 1.04,
+//    5120 (20 row groups leave 8 runs and 96 CUs idle: 401, 16) 1.10; V = 5000,
+//    2048 (18, 1) 0.88, 3072 (28, 1) 1.21, 4096 (28, 2) 0.81, 6144 (48, 2) 1.16;
+//  * several launches, at 19: K = 768, V = 20000, M = 16384 (330, 20) 0.95, 12544
+//    (330, 16) 1.06..1.10; V = 5000, 9216 (61, 3) 1.10.
+bool kr_gemm_head_rows_faster(int M, int N, int K, const kr_half* out, long long ldo) {
+    if ((ldo & 3) != 0 || ((uintptr_t)out & 7) != 0) return M <= kLaunchRows || N >= 4096;
+    if ((2 * ldo) % 4096 == 0) return M <= 1024;
+    if (N < 4096 && M > 4096) return false;
+    if (K < 768 && 2ll * M * ldo > 200000000ll) return false;
+    if (M > kLaunchRows && !(K == 768 && N >= 20000)) return false;
+    const long long tiles = ((M + 255ll) / 256) * ((N + 255) / 256);
+    long long blocks = 0;
+    for (int r0 = 0; r0 < M; r0 += kLaunchRows) {
+        const int runs = column_runs((std::min(M - r0, kLaunchRows) + 255) / 256, N);
+        blocks += ((N + 15) / 16 + runs - 1) / runs + 8;
+    }
+    return 2 * blocks <= (M > kLaunchRows ? 38 : 43) * ((tiles + 255) / 256);
 }
 
 int kr_gemm_head_rows(const kr_half* Af, const kr_half* Wf, int M, int N, int K, kr_half* out,
                       long long ldo, hipStream_t s) {
     KR_REQUIRE(Af && Wf && out, "head: null pointer");
-    KR_REQUIRE(kr_gemm_head_rows_ok(M, N, K), "head: unsupported M=%d N=%d K=%d", M, N, K);
-    KR_REQUIRE(ldo >= N && ldo < (1ll << 24), "head: ldo %lld (N %d)", ldo, N);
+    KR_REQUIRE(kr_gemm_head_rows_ok(M, N, K, ldo), "head: unsupported M=%d N=%d K=%d ldo=%lld", M, N, K, ldo);
     KR_REQUIRE(((uintptr_t)Af & 15) == 0 && ((uintptr_t)Wf & 15) == 0,
                "head: operands must be 16-byte aligned");
-    // one workgroup per CU: as many column runs (whole eights) as the row
-    // groups leave; more than 32 row groups go in several launches
-    constexpr int kRows = 32 * 256;
-    for (int r0 = 0; r0 < M; r0 += kRows) {
-        const int m = M - r0 < kRows ? M - r0 : kRows, mh = (m + 255) / 256, nb = (N + 15) / 16;
-        int ncr = nb < 256 / mh ? nb : 256 / mh;
-        if (ncr >= 8) ncr &= ~7;
+    for (int r0 = 0; r0 < M; r0 += kLaunchRows) {
+        const int m = M - r0 < kLaunchRows ? M - r0 : kLaunchRows, mh = (m + 255) / 256;
+        const int ncr = column_runs(mh, N);
         const kr_half* A = Af + (size_t)r0 * K;
         kr_half* o = out + (size_t)r0 * (size_t)ldo;
         switch (K) {

@@ -1287,8 +1287,8 @@ int kr_impl_embed(const kr_model_weights* m, const int32_t* ids, int M, void* x,
 // logits[M, ld] = fp16(LN_out(x) @ head); xn is an [M, C] fp16 scratch.
 // Up to 512 rows (the decode step) with a fragment-packed head: LN_out writes
 // xn fragment-packed and the small-M head kernel reads it; more rows take
-// kr_head.hip's. Both need xn to hold M rounded up to 16 rows (xn_rows16).
-// Otherwise xn is row-major and the 256 x 256 kernel runs. All follow the
+// kr_head.hip's where it is the faster one. Both need xn to hold M rounded up
+// to 16 rows (xn_rows16). Otherwise xn is row-major and the 256 x 256 kernel runs. All follow the
 // head's one-chain contract (kr_gemm.h), so a row's logits do not depend on
 // the path.
 int kr_impl_head(const kr_model_weights* m, const void* x, int M, void* xn, void* logits,
@@ -1300,7 +1300,8 @@ int kr_impl_head(const kr_model_weights* m, const void* x, int M, void* xn, void
     // 256x128 launch, and one 512-row launch decodes 0.7% faster than the two
     // (B = 512, A B twice on one box).
     const bool small = xn_rows16 && m->headF && kr_gemm_head_small_ok(M, m->V, m->C);
-    const bool rows = xn_rows16 && m->headF && kr_gemm_head_rows_ok(M, m->V, m->C) && ld < (1ll << 24);
+    const bool rows = xn_rows16 && m->headF && kr_gemm_head_rows_ok(M, m->V, m->C, ld) &&
+                      kr_gemm_head_rows_faster(M, m->V, m->C, H(logits), ld);
     LnMixArgs a{};
     a.x = H(x);
     a.ln_w = H(m->ln_out_w);

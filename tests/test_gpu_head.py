@@ -1,4 +1,5 @@
-"""The head's C entry: LN_out scratch in place of its input."""
+"""The head's C entry: LN_out scratch in place of its input, and the row counts
+and strides where its kernels meet."""
 import pytest
 import torch
 
@@ -25,5 +26,28 @@ def test_head_in_place(M):
         ref = _head(P, x, torch.empty_like(x), 1005)
         y = x.clone()
         assert torch.equal(_head(P, y, y, 1005), ref)
+    finally:
+        cpp_path.release_weights(w)
+
+
+# both sides of each line between the register-held rows and the 256 x 256
+# tiles: strides of whole 4096 bytes, few columns, output size at the small
+# widths, row groups that fill the CUs, several launches
+@pytest.mark.parametrize("C,V,ld,Ms", [(256, 2040, 2048, (1024, 1040)), (768, 1000, 1000, (4096, 4112)),
+                                       (512, 5000, 5000, (8192, 8208)), (256, 40000, 40000, (2496, 2512)),
+                                       (768, 5000, 5000, (5120, 6144)), (768, 20000, 20000, (8208,)),
+                                       (256, 4097, 4097, (8208,)), (256, 1001, 1001, (8192, 8208))])
+def test_head_on_both_sides_of_its_lines(C, V, ld, Ms):
+    """The head's kernels share one contract: a row's logits do not depend on
+    the rows around it (here against 512 rows at a time)."""
+    w = synthetic.make_weights(n_layer=1, C=C, F=256, V=V, seed=C + V)
+    P = cpp_path.init_weights(w, "cuda")["prepared"]
+    try:
+        for M in Ms:
+            x = torch.randn((M, C), generator=torch.Generator().manual_seed(M)).half().cuda()
+            got = _head(P, x, torch.empty_like(x), ld)
+            for r in range(0, M, 512):
+                part = x[r:r + 512].contiguous()
+                assert torch.equal(got[r:r + 512], _head(P, part, torch.empty_like(part), ld)), (M, r)
     finally:
         cpp_path.release_weights(w)
