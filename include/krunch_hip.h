@@ -144,6 +144,11 @@ int kr_softmax_cdf_decode(const uint16_t* logits, int B, int V, long long ld,
 /* W [K, N] (row stride ldw) -> Wt [N, K] (row stride ldt), fp16. */
 int kr_transpose_f16(const uint16_t* W, long long ldw, int K, int N, uint16_t* Wt,
                      long long ldt, void* stream);
+/* The same with Wf, the fragment-packed copy of Wt (kr_pack_fragments below:
+ * kr_fragment_bytes(N, K) bytes, 16-byte aligned), in the same launch;
+ * K % 32 == 0. */
+int kr_transpose_pack_f16(const uint16_t* W, long long ldw, int K, int N, uint16_t* Wt,
+                          long long ldt, uint16_t* Wf, void* stream);
 
 /* replaces krunch_ac_cuda.det_matmul (layer_cpp.cpp:728-822, det_matmul_tc*.cu):
  * out = epilogue(x [M,K] @ W) with W given as Wt [N, ldw]. epilogue: 0 fp32 out,

@@ -64,6 +64,7 @@ _SIGS = {
     "kr_softmax_cdf_decode": ([P, I, I, LL, P, U32, P, P, P, P, P, LL, P, P, I, P], I),
     # GEMM / layers / model
     "kr_transpose_f16": ([P, LL, I, I, P, LL, P], I),
+    "kr_transpose_pack_f16": ([P, LL, I, I, P, LL, P, P], I),
     "kr_det_matmul": ([P, I, I, P, LL, I, P, LL, I, P, P, P], I),
     "kr_fragment_bytes": ([I, I], ctypes.c_size_t),
     "kr_pack_fragments": ([P, LL, I, I, P, P], I),

@@ -22,7 +22,7 @@ ARCH = os.environ.get("KRUNCH_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = ["kr_rc.hip", "kr_cdf.hip", "kr_gemm.hip", "kr_quant.hip", "kr_layer.hip", "kr_engine.hip",
            "kr_wide.hip", "kr_mid.hip", "kr_wkv.hip",
-           "kr_step.hip", "kr_head.hip"]
+           "kr_step.hip", "kr_head.hip", "kr_pack.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -176,29 +176,31 @@ def softmax_probs(logits):
 _WT_CACHE: dict = {}
 
 
-def _wt(W):
-    """Transposed copy of a [K, N] weight, cached per live tensor object and version."""
-    return _wt_wf(W)[0]
-
-
-def _wt_wf(W, frag=False):
-    """The same with, on request, the fragment-packed copy that the layer's
-    products read (kept in the same entry; else None). frag needs K % 32 == 0.
-    Copies made while the stream is capturing are written when the graph runs,
-    not now, so they serve that call only."""
+def _copies(W, frag):
+    """Device copies of a [K, N] weight, kept per live tensor object and
+    version: pointers to the transposed one and, on request, to the
+    fragment-packed one that the layer's products read (frag needs
+    K % 32 == 0), and the tensors that hold them. Copies made while the stream
+    is capturing are written when the graph runs, not now, so they serve that
+    call only."""
     key = id(W)
-    hit = _WT_CACHE.get(key)
-    known = hit
+    hit = known = _WT_CACHE.get(key)
     if hit is None or hit[0]() is not W or hit[1] != W._version:
         K, N = W.shape
-        wt = torch.empty((N, K), dtype=torch.float16, device=W.device)
-        _lib.call("kr_transpose_f16", W.data_ptr(), N, K, N, wt.data_ptr(), K, _lib.stream_ptr())
-        hit = (weakref.ref(W, lambda _r, k=key: _WT_CACHE.pop(k, None)), W._version, wt, None)
-    if frag and hit[3] is None:
-        N, K = hit[2].shape
-        wf = torch.empty(_lib.lib().kr_fragment_bytes(N, K), dtype=torch.uint8, device=W.device)
-        _lib.call("kr_pack_fragments", hit[2].data_ptr(), K, N, K, wf.data_ptr(), _lib.stream_ptr())
-        hit = hit[:3] + (wf,)
+        rows = (N + 15) // 16 * 16 if frag else 0
+        buf = torch.empty((N + rows) * K, dtype=torch.float16, device=W.device)
+        wt = buf.data_ptr()
+        wf = wt + 2 * N * K if frag else None
+        if frag:
+            _lib.call("kr_transpose_pack_f16", W.data_ptr(), N, K, N, wt, K, wf, _lib.stream_ptr())
+        else:
+            _lib.call("kr_transpose_f16", W.data_ptr(), N, K, N, wt, K, _lib.stream_ptr())
+        hit = (weakref.ref(W, lambda _r, k=key: _WT_CACHE.pop(k, None)), W._version, wt, wf, (buf,))
+    elif frag and hit[3] is None:
+        K, N = W.shape
+        buf = torch.empty((N + 15) // 16 * 16 * K, dtype=torch.float16, device=W.device)
+        _lib.call("kr_pack_fragments", hit[2], K, N, K, buf.data_ptr(), _lib.stream_ptr())
+        hit = (*hit[:3], buf.data_ptr(), (*hit[4], buf))
     if hit is not known and not torch.cuda.is_current_stream_capturing():
         _WT_CACHE[key] = hit
     return hit[2:]
@@ -214,7 +216,8 @@ def det_matmul(x, W, out_dtype=None):
     dtype = out_dtype or torch.float16
     out = torch.empty((M, N), dtype=dtype, device=x.device)
     ep = 0 if dtype == torch.float32 else 1
-    _lib.call("kr_det_matmul", x.data_ptr(), M, K, _wt(W).data_ptr(), K, N, out.data_ptr(), N,
+    wt, _, _keep = _copies(W, False)
+    _lib.call("kr_det_matmul", x.data_ptr(), M, K, wt, K, N, out.data_ptr(), N,
               ep, None, None, _lib.stream_ptr())
     return out
 
@@ -246,9 +249,9 @@ def _layer_struct(x, att_xx, aa, bb, pp, ffn_xx, ln1_w, ln1_b, tm_k, tm_v, tm_r,
     def wt(m, k, n):
         _cuda(m, torch.float16, "weight")
         _check(tuple(m.shape) == (k, n), f"weight must be [{k}, {n}], got {tuple(m.shape)}")
-        t = _wt_wf(m, frag=True)
-        keep.extend(t)
-        return t[0].data_ptr(), t[1].data_ptr()
+        wt_ptr, wf_ptr, held = _copies(m, True)
+        keep.append(held)
+        return wt_ptr, wf_ptr
 
     L = _lib.KrLayerWeights()
     L.ln1_w, L.ln1_b, L.tm_k, L.tm_v, L.tm_r = map(h, (ln1_w, ln1_b, tm_k, tm_v, tm_r))
@@ -278,7 +281,9 @@ def rwkv4_layer_step_cpp(x, att_xx, aa, bb, pp, ffn_xx, ln1_w, ln1_b, tm_k, tm_v
     """One RWKV-4 layer over x [B, T, C] fp16 (any B, T); state mutated in
     place; returns the new x (layer_cpp.cpp:456-637). `time_decay` is
     w = -exp(raw) as the reference's rwkv loader passes it (wkv_kernel.cu:41-45).
-    Matrices are [in, out] (y = x @ W)."""
+    Matrices are [in, out] (y = x @ W); the first call on a weight makes a
+    transposed and a fragment-packed copy of it, which live as long as the
+    tensor (4 bytes per parameter) and are remade after an in-place change."""
     args = (x, att_xx, aa, bb, pp, ffn_xx, ln1_w, ln1_b, tm_k, tm_v, tm_r, time_decay,
             time_first, Kw, Vw, Rw, Ow, ln2_w, ln2_b, ffn_tm_k, ffn_tm_r, ffn_Kw, ffn_Vw, ffn_Rw)
     L, C, F, _keep = _layer_struct(*args)
@@ -312,8 +317,8 @@ def rwkv4_layer_step_cpp_graphed(layer_id, x_buf, x_out_buf, att_xx, aa, bb, pp,
     state exactly once; the reference's warm-up runs and capture advance it
     three times on the first call (cpp_path.py:369-384 records that as a bug).
     The graph also keys on the buffer addresses and shapes, so new buffers get
-    a new graph instead of a stale replay. The graph runs on the transposed
-    weight copies made at capture time: after an in-place change of a
+    a new graph instead of a stale replay. The graph runs on the weight copies
+    (transposed, fragment-packed) made at capture time: after an in-place change of a
     weight tensor (same address), call clear_layer_graph_cache()."""
     _cuda(x_buf, torch.float16, "x_buf")
     _cuda(x_out_buf, torch.float16, "x_out_buf")

@@ -1,8 +1,9 @@
 """The layer op's weight copies (transposed and fragment-packed, kept per
-weight tensor): calls inside a stream capture."""
+weight tensor): how they are made, and calls inside a stream capture."""
 import pytest
 import torch
 
+from krunch_amd import _lib
 from krunch_amd import krunch_ac_hip as ops
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +61,19 @@ def test_layer_captured_on_new_weights(B, T, warm):
         for a, b in zip(st, ref_st):
             assert torch.equal(a, b)
         assert torch.equal(_call(d, _state(B)), ref)
+
+
+# whole and partial tiles of 32 and blocks of 16 columns, one k block and
+# several, strides past the row ends
+@pytest.mark.parametrize("K,N,ldw,ldt", [(32, 1, 1, 32), (64, 15, 15, 64), (96, 16, 20, 96), (256, 17, 17, 264),
+                                         (32, 33, 40, 32), (768, 3072, 3072, 768)])
+def test_transpose_pack_equals_the_two_calls(K, N, ldw, ldt):
+    W = torch.randn(K, ldw, generator=torch.Generator().manual_seed(K + N)).half().cuda()
+    s = _lib.stream_ptr()
+    n = _lib.lib().kr_fragment_bytes(N, K) // 2
+    wt, ref = (torch.full((N, ldt), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
+    wf, ref_f = (torch.full((n,), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
+    _lib.call("kr_transpose_pack_f16", W.data_ptr(), ldw, K, N, wt.data_ptr(), ldt, wf.data_ptr(), s)
+    _lib.call("kr_transpose_f16", W.data_ptr(), ldw, K, N, ref.data_ptr(), ldt, s)
+    _lib.call("kr_pack_fragments", ref.data_ptr(), ldt, N, K, ref_f.data_ptr(), s)
+    assert torch.equal(wt, ref) and torch.equal(wf, ref_f)
