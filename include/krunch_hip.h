@@ -352,6 +352,11 @@ int kr_embed(const kr_model_weights* m, const int32_t* ids, int M, void* x, void
  * same bits for any M, with or without headF (decode and compress agree). */
 int kr_head_logits(const kr_model_weights* m, const void* x, int M, void* xn, void* logits,
                    long long ld, void* stream);
+/* The same with xn (not x) holding M rounded up to 16 rows: the heads that read
+ * fragment-packed rows, which kr_head_logits gives whole 16-row blocks only,
+ * then take any M. */
+int kr_head_logits_rows16(const kr_model_weights* m, const void* x, int M, void* xn, void* logits,
+                          long long ld, void* stream);
 
 /* One packed compress window for B streams x T tokens (rows b*T + t): embed,
  * layers, then per block of head_rows rows head logits -> softmax -> symbol

@@ -92,6 +92,7 @@ _SIGS = {
     "kr_forward_layers": ([ctypes.POINTER(KrModelWeights), P, I, I, P, P, SZ, P], I),
     "kr_embed": ([ctypes.POINTER(KrModelWeights), P, I, P, P], I),
     "kr_head_logits": ([ctypes.POINTER(KrModelWeights), P, I, P, P, LL, P], I),
+    "kr_head_logits_rows16": ([ctypes.POINTER(KrModelWeights), P, I, P, P, LL, P], I),
     "kr_compress_window": ([ctypes.POINTER(KrModelWeights), P, P, I, I, P, P, P, SZ, P, LL, I,
                             P, I, P], I),
     "kr_decode_step": ([ctypes.POINTER(KrModelWeights), I, P, P, P, P, SZ, P, LL, P, U32, P, P,

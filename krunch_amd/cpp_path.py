@@ -119,16 +119,16 @@ def forward_packed_batched(weights: dict, input_ids, state: State) -> torch.Tens
     assert state.B == B, f"state holds {state.B} streams, input has {B}"
     _check_ids(ids, P.V)
     M = B * T
-    M16 = (M + 15) // 16 * 16      # whole row blocks for the head, whose spare rows are dropped
-    x = torch.empty((M16, P.C), dtype=torch.float16, device=P.device)
+    x = torch.empty((M, P.C), dtype=torch.float16, device=P.device)
     s = _lib.stream_ptr()
     _lib.call("kr_embed", P.ptr, ids.data_ptr(), M, x.data_ptr(), s)
     ws, nbytes = workspace(weights, M)
     _lib.call("kr_forward_layers", P.ptr, x.data_ptr(), B, T, state.ptr, ws.data_ptr(), nbytes, s)
-    xn = torch.empty_like(x)
-    logits = torch.empty((M16, P.V), dtype=torch.float16, device=P.device)
-    _lib.call("kr_head_logits", P.ptr, x.data_ptr(), M16, xn.data_ptr(), logits.data_ptr(), P.V, s)
-    return logits[:M]
+    xn = torch.empty(((M + 15) // 16 * 16, P.C), dtype=torch.float16, device=P.device)
+    logits = torch.empty((M, P.V), dtype=torch.float16, device=P.device)
+    _lib.call("kr_head_logits_rows16", P.ptr, x.data_ptr(), M, xn.data_ptr(), logits.data_ptr(),
+              P.V, s)
+    return logits
 
 
 def forward_packed(weights: dict, input_ids, state: State) -> torch.Tensor:
@@ -171,9 +171,9 @@ def forward_stepped_graphed(weights: dict, last_token: int, state: State) -> tor
     if hit is None:
         dev = P.device
         ids = torch.zeros(1, dtype=torch.int32, device=dev)
-        x = torch.zeros((16, P.C), dtype=torch.float16, device=dev)
+        x = torch.empty((1, P.C), dtype=torch.float16, device=dev)
         xn = torch.empty((16, P.C), dtype=torch.float16, device=dev)
-        logits = torch.empty((16, P.V), dtype=torch.float16, device=dev)   # row 0 and spare rows
+        logits = torch.empty((1, P.V), dtype=torch.float16, device=dev)
         ws, nbytes = workspace(weights, 16)
         ws = ws.clone()        # private to the graph: the shared workspace may grow
         torch.cuda.synchronize(dev)
@@ -183,8 +183,8 @@ def forward_stepped_graphed(weights: dict, last_token: int, state: State) -> tor
             _lib.call("kr_embed", P.ptr, ids.data_ptr(), 1, x.data_ptr(), s)
             _lib.call("kr_forward_layers", P.ptr, x.data_ptr(), 1, 1, state.ptr, ws.data_ptr(),
                       nbytes, s)
-            _lib.call("kr_head_logits", P.ptr, x.data_ptr(), 16, xn.data_ptr(), logits.data_ptr(),
-                      P.V, s)
+            _lib.call("kr_head_logits_rows16", P.ptr, x.data_ptr(), 1, xn.data_ptr(),
+                      logits.data_ptr(), P.V, s)
         # the entry holds the weights bundle, so its id cannot be reused for
         # another bundle while the graph (which points into it) is cached
         hit = (graph, ids, x, xn, logits, ws, weights)
@@ -195,7 +195,7 @@ def forward_stepped_graphed(weights: dict, last_token: int, state: State) -> tor
         raise ValueError(f"token id out of range [0, {P.V})")
     ids.fill_(tok)
     graph.replay()
-    return logits[0].clone()
+    return logits.reshape(-1).clone()
 
 
 def clear_graph_cache():

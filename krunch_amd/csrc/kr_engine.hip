@@ -146,6 +146,12 @@ int kr_head_logits(const kr_model_weights* m, const void* x, int M, void* xn, vo
     return kr_impl_head(m, x, M, xn, logits, ld, kr_stream(stream), M % 16 == 0 && xn != x);
 }
 
+int kr_head_logits_rows16(const kr_model_weights* m, const void* x, int M, void* xn, void* logits,
+                          long long ld, void* stream) {
+    KR_REQUIRE(m && x && xn && logits && xn != x && M >= 0 && ld >= m->V, "kr_head_logits_rows16: bad args");
+    return kr_impl_head(m, x, M, xn, logits, ld, kr_stream(stream), true);
+}
+
 int kr_compress_window(const kr_model_weights* m, const int32_t* inputs, const int32_t* targets,
                        int B, int T, void* state, void* x, void* ws, size_t ws_bytes,
                        void* logits, long long ld, int head_rows, uint32_t* pairs,

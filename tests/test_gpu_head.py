@@ -51,3 +51,27 @@ def test_head_on_both_sides_of_its_lines(C, V, ld, Ms):
                 assert torch.equal(got[r:r + 512], _head(P, part, torch.empty_like(part), ld)), (M, r)
     finally:
         cpp_path.release_weights(w)
+
+
+# one row, around a 16-row block, around the decode head's 512 rows; widths
+# with and without fragment-packed heads
+@pytest.mark.parametrize("C", [256, 1024])
+@pytest.mark.parametrize("M", [1, 15, 17, 511, 513, 700])
+def test_logits_hold_their_rows_only(C, M):
+    """Packed and stepped logits own M rows and no more, equal to the head's
+    over rows of their own."""
+    w = synthetic.make_weights(n_layer=1, C=C, F=256, V=1003, seed=M)
+    W = cpp_path.init_weights(w, "cuda")
+    try:
+        ids = torch.from_numpy(synthetic.zipf_tokens(1, M, V=1003))
+        got = cpp_path.forward_packed_batched(W, ids, cpp_path.fresh_state(W))
+        assert got.shape == (M, 1003) and got.untyped_storage().nbytes() == 2 * M * 1003
+        st = cpp_path.fresh_state(W)
+        for t in range(min(M, 3)):
+            one = cpp_path.forward_stepped(W, int(ids[0, t]), st)
+            assert torch.equal(one, got[t]) and one.untyped_storage().nbytes() == 2 * 1003
+        st.reset()
+        assert torch.equal(cpp_path.forward_stepped_graphed(W, int(ids[0, 0]), st), got[0])
+    finally:
+        cpp_path.clear_graph_cache()
+        cpp_path.release_weights(w)
