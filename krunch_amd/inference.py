@@ -106,9 +106,13 @@ def decode_header(data: bytes) -> dict:
             "n_chunks": n_chunks, "crc32": crc}
 
 
-# What a window costs beside its rows, in rows: one layer takes 146 us at 1024
-# rows and 493 at 8192 on MI355X, so a window's 12 layers cost about 1.1 ms + 0.58 us
-# per row.
+# What a further window costs beside its rows, in rows. A window of 512..20000
+# rows (layers, head and CDF) takes about 0.70 ms + 0.55 us per row on MI355X, so
+# some 1300 rows, and a second window also costs the encoder's second stream, the
+# state's copy and the gaps between windows. Measured over 23 sets of ragged
+# streams (2..200 streams of 50..16100 tokens), both codecs, time against this
+# constant's: 500 rows 1.089, 800 1.050, 1250 1.025, 1600 1.010, 2500 1.000, 4500
+# 1.001.
 WINDOW_ROWS = 2000
 
 
