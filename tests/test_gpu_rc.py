@@ -240,3 +240,27 @@ def test_wave_encoder_batches_and_pending_runs(N):
         ref = orc.encode(cdf, sym)
         assert _gpu_encode(cdf, sym) == ref
         assert _gpu_encode(cdf, sym, chunks=min(3, N)) == ref
+
+
+# past 256 complements carried into the run's last batch, of one symbol to a
+# whole batch, with and without a partial byte before it
+@pytest.mark.parametrize("first", [0, 3])
+@pytest.mark.parametrize("last", [1, 2, 17, 63, 64])
+def test_run_that_ends_in_a_serially_written_batch(first, last):
+    """Symbols that only add complements fill whole batches, so the last one
+    carries more than the bit window holds and goes out serially; the run's
+    tail follows straight after it. Bytes and state as the oracle's, in one
+    call and with another run behind it."""
+    q = 1 << 22
+    cdf3 = np.array([0, q, 3 * q, 4 * q], dtype=np.uint32)
+    rng = np.random.default_rng(100 * first + last)
+    tail = rng.integers(0, 3, last)
+    tail[0] = 2 * (last % 2)                                # the first of them emits
+    ends = np.where(rng.integers(0, 2, first) == 0, 0, 2)   # a few bits before the complements
+    sym = np.concatenate([ends, np.ones(384 - first, dtype=np.int64), tail]).astype(np.int32)
+    cdf = np.tile(cdf3, (len(sym), 1))
+    ref = orc.encode(cdf, sym)
+    assert _gpu_encode(cdf, sym) == ref
+    more = np.concatenate([sym, sym]).astype(np.int32)
+    assert _gpu_encode(np.tile(cdf3, (len(more), 1)), more, chunks=2) == orc.encode(
+        np.tile(cdf3, (len(more), 1)), more)

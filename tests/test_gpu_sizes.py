@@ -25,7 +25,7 @@ def _weights(C):
 @pytest.mark.parametrize("C", [256, 512, 1024])
 def test_width_packed_equals_stepped(C, w8a8):
     """B = 3 streams over 40 tokens (small-M kernels on both sides) and 2
-    streams over 600 (packed on the tiled kernel): packed == stepped, state
+    streams over 600 (packed on the register-fed kernel): packed == stepped, state
     included; fp16 logits within 1e-2 of the fp32 oracle."""
     w16 = _weights(C)
     W = cpp_path.init_weights(w16, "cuda", w8a8=w8a8)

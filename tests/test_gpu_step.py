@@ -114,3 +114,41 @@ def test_step_timing_leaves_the_launches_as_they_are(B, w8a8):
                                        (1024, True, (96, 97))])
 def test_stepped_equals_packed_at_the_lines(C, w8a8, Bs):
     test_stepped_equals_packed(C, Bs, w8a8)
+
+
+def test_decode_run_refuses_a_capturing_stream():
+    """With use_graph the run waits for its steps on the caller's stream; on
+    one that is being captured it is an error, and the capture goes on."""
+    w = synthetic.make_weights(n_layer=2, V=300, seed=4)
+    P = cpp_path.init_weights(w, "cuda")["prepared"]
+    B, dev = 3, dict(device="cuda")
+    syms = torch.full((B,), 5, dtype=torch.int32, **dev)
+    bits = torch.zeros(64, dtype=torch.uint8, **dev)
+    ac = torch.zeros((B, 4), dtype=torch.uint32, **dev)
+    st = cpp_path.fresh_state_batched({"prepared": P}, B)
+    x = torch.zeros((B, P.C), dtype=torch.float16, **dev)
+    ws = torch.empty(_lib.lib().kr_decode_workspace_bytes(B, 1, P.C, P.F), dtype=torch.uint8, **dev)
+    logits = torch.empty((B, P.V), dtype=torch.float16, **dev)
+    before = st.buf.clone()
+    y = torch.zeros(4, **dev)
+    torch.cuda.synchronize()
+
+    def run():
+        _lib.call("kr_decode_run", P.ptr, B, st.ptr, syms.data_ptr(), x.data_ptr(), ws.data_ptr(),
+                  ws.numel(), logits.data_ptr(), P.V, bits.data_ptr(), 64, None, None, ac.data_ptr(),
+                  None, 0, None, None, 24, 2, 1, 1, _lib.stream_ptr())
+
+    try:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            y.add_(1.0)
+            with pytest.raises(_lib.KrunchError, match="captured"):
+                run()
+            y.add_(1.0)
+        for i in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            assert y.tolist() == [2.0 * (i + 1)] * 4
+        assert torch.equal(st.buf, before) and syms.tolist() == [5] * B
+    finally:
+        cpp_path.release_weights(w)
