@@ -243,7 +243,8 @@ typedef struct kr_layer_weights {
     const void *fVt;                      /* fp16 [C, F] */
     const void *fRt;                      /* fp16 [C, C] */
     /* Fragment-packed copies of the seven matrices above (kr_pack_fragments),
-     * read by the small-M (B*T <= 512) path; all NULL = use the row-major ones. */
+     * read up to 512 rows (B*T) and, by the register-fed products, up to 1536
+     * .. 2304 by width and codec; all NULL = use the row-major ones. */
     const void *Kf, *Vf, *Rf, *Of, *fKf, *fVf, *fRf;
     /* w8a8 codec: int8 copies of the seven matrices; the
      * layer then runs its GEMMs on int8 MFMA with per-token activation
@@ -257,8 +258,9 @@ typedef struct kr_model_weights {
     const void *ln_out_w, *ln_out_b;      /* fp16 [C] */
     const void* headT;                    /* fp16 [V, C] */
     const kr_layer_weights* layers;       /* host array, n_layer entries */
-    /* Fragment-packed copy of headT (kr_pack_fragments), read by the decode
-     * head (M <= 512 rows, C <= 768); NULL = the row-major head. */
+    /* Fragment-packed copy of headT (kr_pack_fragments), read for C <= 768 by
+     * the decode head (M <= 512 rows) and by the register-held rows above that;
+     * NULL = the row-major head. */
     const void* headF;
 } kr_model_weights;
 

@@ -22,8 +22,8 @@ struct kr_gemm_args {
     const kr_half* res;   // [M, N] stride ldo (RESID, GATED); may alias out
     const kr_half* gate;  // [M, N] stride ldo (GATED)
     int M, N, K;
-    const kr_half* Wf;  // W^T fragment-packed (kr_frag_index), or null; small-M path only
-    int a_frag;         // A is fragment-packed (small-M path only; needs Wf)
+    const kr_half* Wf;  // W^T fragment-packed (kr_frag_index), or null; read when a_frag
+    int a_frag;         // A is fragment-packed (M <= KR_GEMM_MID_M, int8 KR_GEMM_MID_M_I8; needs Wf)
     int out_frag;       // fp16 output written fragment-packed as a K = N operand
     // w8a8: A and W^T hold int8 (pointers reinterpreted; lda/ldw in bytes),
     // acc = exact int32 sum, value = (float(acc) * sa[m]) * sw[n], then the epilogue.
@@ -158,8 +158,6 @@ struct kr_panel_timing {
     hipEvent_t start, stop;
 };
 kr_panel_timing kr_gemm_take_timing(int groups, int waves);
-// Several products; on the small-M path those sharing M and K run in one
-// launch (independent outputs), otherwise they are launched in order.
 // Width (in 16-column panels) of the column groups the small-M fragment
 // kernel uses for these jobs launched together. When a job has a multiple of 8
 // groups, XCD x takes its groups x, x + 8, ... (workgroups are dealt to the
@@ -167,11 +165,14 @@ kr_panel_timing kr_gemm_take_timing(int groups, int waves);
 // XCD's L2 ahead of the launch.
 int kr_gemm_panel_ns(const kr_gemm_args* jobs, int njobs);
 
+// Several products; those sharing M and K run in one launch on the small-M path
+// and, with fragment-packed operands, up to KR_GEMM_MID_M rows (int8
+// KR_GEMM_MID_M_I8; independent outputs); otherwise they are launched in order.
 int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* epilogues, int njobs,
                          hipStream_t stream, const kr_row_copy* copy = nullptr);
 
 // The head (logits = fp16(LN_out(x) @ head)) has a reduction contract of
-// its own, which the two head kernels below share and no other product uses:
+// its own, which the three head kernels below share and no other product uses:
 //   acc = chain of v_mfma_f32_16x16x32_f16 over k = 0, 32, ..., K - 32 from
 //         zero (one chain, no slice partials), out = fp16(acc).
 // A row's logits are therefore the same bits for any M and either kernel.

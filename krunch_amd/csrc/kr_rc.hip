@@ -1,10 +1,12 @@
 // Range-coder kernels and their C-ABI entry points.
 //
-// One lane per independent stream; the coder is serial within a stream. The
-// entry points keep the reference's argument meaning and state layout
-// (krunch_ac/cuda/main.cpp encode_step / decode_step and their _batched
-// forms; encode_kernel.cu, decode_kernel.cu) and add buffer bounds: output
-// writes stop at out_cap, input reads past a stream's limit return zeros.
+// The coder is serial within a stream. Runs of symbols (kr_encode_step,
+// kr_encode_pairs_batched) are encoded by one wave per stream, the lockstep
+// calls of one symbol per stream by one lane per stream. The entry points keep
+// the reference's argument meaning and state layout (krunch_ac/cuda/main.cpp
+// encode_step / decode_step and their _batched forms; encode_kernel.cu,
+// decode_kernel.cu) and add buffer bounds: output writes stop at out_cap, input
+// reads past a stream's limit return zeros.
 #include "kr_rc_device.h"
 
 namespace {

@@ -1,4 +1,5 @@
-// Device-side range coder: one lane owns one independent stream.
+// Device-side range coder, one lane per stream (kr_rc.hip has the wave form of
+// the encoder).
 //
 // Bit-exact with the spec krunch_ac/cpu_reference.py:91-234: 32-bit
 // low/high, E1/E2/E3 renormalisation, pending (E3) bits emitted as
