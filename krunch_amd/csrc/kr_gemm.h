@@ -103,9 +103,7 @@ inline int kr_gemm_mid_rows(int C, bool i8) {
     return C <= 512 ? KR_GEMM_MID_M : (C <= 768 ? 2176 : 1856);
 }
 
-// A row copy that rides along in a small-M product launch (8-byte units,
-// 8-byte aligned): the carried rows a fused LN-mix left beside the state it
-// read (kr_step.hip).
+// A row copy that rides along in a product launch (8-byte units; kr_panel.h).
 struct kr_row_copy {
     const uint2* src;
     uint2* dst;
@@ -118,7 +116,6 @@ struct kr_gemm_multi {
     int ep[KR_GEMM_MAX_JOBS];
     int tiles[KR_GEMM_MAX_JOBS];
     int njobs;
-    kr_row_copy copy;          // n = 0: none
     // decode-step timing (null otherwise): wave w of workgroup b stores its
     // start and end times (the 100 MHz steady counter) at stamps[16 b + w]
     unsigned long long* stamps;
@@ -131,16 +128,17 @@ struct kr_gemm_multi {
 //   acc = P_0; acc = acc + P_1; ...; acc = acc + P_{S-1}   (fp32 adds, in order),
 // then the epilogue. A row therefore gets identical bits for any M. The int8
 // path accumulates exactly in int32, so any order gives the same bits.
-// copy (nullable): done in the same launch; fragment-packed small-M products only.
-int kr_gemm_launch(const kr_gemm_args& g, int epilogue, hipStream_t stream,
-                   const kr_row_copy* copy = nullptr);
+int kr_gemm_launch(const kr_gemm_args& g, int epilogue, hipStream_t stream);
+// What every launch checks first.
+int kr_gemm_check(const kr_gemm_args& g, int epilogue);
 
 // Kernel timing for the decode-step profiler: the next small-M panel launch
 // on this host thread (kr_gemm_launch / kr_gemm_launch_multi choosing
-// gemm_panel_kernel, or kr_step_launch_rk) with at most max_groups workgroups
-// gets `stamps` (2 x KR_STAMP_WAVES x max_groups u64, see kr_gemm_multi) and
-// stores each wave's start and end times there, also when it is captured in a
-// graph (then at every replay). Arm with a buffer, disarm with nullptr.
+// gemm_panel_kernel, or kr_step.hip's products but K/V/R) with at most
+// max_groups workgroups gets `stamps` (2 x KR_STAMP_WAVES x max_groups u64, see
+// kr_gemm_multi) and stores each wave's start and end times there, also when it
+// is captured in a graph (then at every replay). Arm with a buffer, disarm with
+// nullptr.
 // kr_gemm_timed_launch_taken(): the grid size of the panel launch that took
 // the buffer since it was armed; 0 if none came; minus the grid size if one
 // came with more than max_groups workgroups (it ran untimed).
@@ -169,7 +167,7 @@ int kr_gemm_panel_ns(const kr_gemm_args* jobs, int njobs);
 // and, with fragment-packed operands, up to KR_GEMM_MID_M rows (int8
 // KR_GEMM_MID_M_I8; independent outputs); otherwise they are launched in order.
 int kr_gemm_launch_multi(const kr_gemm_args* jobs, const int* epilogues, int njobs,
-                         hipStream_t stream, const kr_row_copy* copy = nullptr);
+                         hipStream_t stream);
 
 // The head (logits = fp16(LN_out(x) @ head)) has a reduction contract of
 // its own, which the three head kernels below share and no other product uses:

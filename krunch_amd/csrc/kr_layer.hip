@@ -783,12 +783,12 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
         KR_TRY(ph.mark(2));
         KR_TRY(ph.mark(3));
         const kr_row_copy att = carried_rows(w.kx, st.att_xx, M, C), ffn = carried_rows(w.fkx, st.ffn_xx, M, C);
-        KR_TRY(kr_gemm_launch(gemm_q8_q16(w.ry, M, C, Q.O, C, x, x), KR_EP_RESID, s, &att));
+        KR_TRY(kr_step_launch_product(gemm_q8_q16(w.ry, M, C, Q.O, C, x, x), KR_EP_RESID, att, s));
         KR_TRY(ph.mark(4));
         KR_TRY(ph.mark(5));
         KR_TRY(kr_step_launch_rk(C, true, step_rk_args(L, x, M, F, st, w), s));
         KR_TRY(ph.mark(6));
-        KR_TRY(kr_gemm_launch(gemm_q8_q16(w.kf, M, F, Q.fV, C, x, x, w.rf), KR_EP_GATED, s, &ffn));
+        KR_TRY(kr_step_launch_product(gemm_q8_q16(w.kf, M, F, Q.fV, C, x, x, w.rf), KR_EP_GATED, ffn, s));
         return ph.mark(7);
     }
     LnMixArgs a{};
@@ -896,12 +896,12 @@ int layer_step_fused(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
         KR_TRY(ph.mark(2));
         KR_TRY(ph.mark(3));
         const kr_row_copy att = carried_rows(w.kx, st.att_xx, M, C), ffn = carried_rows(w.fkx, st.ffn_xx, M, C);
-        KR_TRY(kr_gemm_launch(gemm_args(w.ry, M, C, L.Ot, C, x, x, nullptr, L.Of, true), KR_EP_RESID, s, &att));
+        KR_TRY(kr_step_launch_product(gemm_args(w.ry, M, C, L.Ot, C, x, x, nullptr, L.Of, true), KR_EP_RESID, att, s));
         KR_TRY(ph.mark(4));
         KR_TRY(ph.mark(5));
         KR_TRY(kr_step_launch_rk(C, false, step_rk_args(L, x, M, F, st, w), s));
         KR_TRY(ph.mark(6));
-        KR_TRY(kr_gemm_launch(gemm_args(w.kf, M, F, L.fVt, C, x, x, w.rf, L.fVf, true), KR_EP_GATED, s, &ffn));
+        KR_TRY(kr_step_launch_product(gemm_args(w.kf, M, F, L.fVt, C, x, x, w.rf, L.fVf, true), KR_EP_GATED, ffn, s));
         return ph.mark(7);
     }
     // Weights the next products read, staged into their XCDs' L2 by the

@@ -5,16 +5,18 @@
 // Whether a stepped layer of M streams takes them: beyond, the LN that every
 // column group repeats (C / 16 groups of C values per row) costs more than the
 // launches it saves. Measured on MI355X, one step of 12 layers, F = 4 C, us,
-// six launches per layer / four. fp16: C = 256, M = 16 210 / 196, 160 274 / 223;
-// 512, 16 266 / 235, 160 344 / 275; 768, 16 292 / 272, 128 370 / 324, 144
-// 373 / 374, 160 376 / 379; 1024, 8 332 / 316, 48 352 / 347, 64 379 / 384, 96
-// 408 / 434, 128 437 / 517. w8a8, whose rows are quantised as well: C = 256, 12
-// 240 / 231, 16 240 / 261, 96 263 / 269, 97 301 / 271 (the panel products'
-// tiles change there), 128 304 / 278; 512, 16 302 / 288, 128 354 / 311; 768, 16
-// 327 / 325, 128 399 / 361; 1024, 16 362 / 350, 96 421 / 389, 112 435 / 453.
-// (decode runs of 136..160 streams, C = 768, fp16: 1-2 % faster with six). The
-// limits at C <= 512 (fp16) and 512..768 (w8a8) are the last rows measured
-// ahead, not crossovers.
+// six launches per layer / four. fp16: C = 256, M = 16 211 / 191, 160 279 / 214;
+// 512, 16 270 / 224, 160 345 / 268; 768, 16 297 / 265, 128 377 / 316, 144
+// 386 / 368, 160 384 / 376; 1024, 8 343 / 311, 48 357 / 341, 64 386 / 380, 96
+// 403 / 435, 128 429 / 524. w8a8, whose rows are quantised as well: C = 256, 12
+// 239 / 224, 16 243 / 254, 96 267 / 263, 97 297 / 263 (the panel products'
+// tiles change there), 128 305 / 270; 512, 16 306 / 280, 128 357 / 301; 768, 16
+// 327 / 317, 128 401 / 354; 1024, 16 364 / 343, 96 428 / 382, 112 443 / 443.
+// In a decode run of 144 streams (C = 768), whose logits and symbols come
+// between the steps, four are 2 % ahead in fp16 and 1 % behind in w8a8; of 160,
+// 2 % behind in both. Within 2 % the order differs between builds, so no line
+// goes by that. The limits at C <= 512 (fp16) and 512 (w8a8) are the last rows
+// measured ahead, not crossovers.
 inline bool kr_step_fuse_ok(int C, int M, bool i8) {
     if (i8) return C <= 256 ? M <= 12 || (M > 96 && M <= 128) : M <= (C <= 768 ? 128 : 96);
     return M <= (C <= 512 ? 160 : (C <= 768 ? 128 : 48));
@@ -56,3 +58,6 @@ struct kr_step_rk {
 
 int kr_step_launch_kvr(int C, bool i8, const kr_step_kvr& a, hipStream_t s);
 int kr_step_launch_rk(int C, bool i8, const kr_step_rk& a, hipStream_t s);
+// The layer's O and V products (one fragment-packed product, w8a8: of fp16 rows
+// quantised on load), with the carried rows copied in the same launch.
+int kr_step_launch_product(const kr_gemm_args& g, int epilogue, const kr_row_copy& copy, hipStream_t s);

@@ -12,22 +12,23 @@
 // 0.13 us of issue per row, which is what bounds the range of M.
 //
 // The carried row (state) is read by every column group, so the new one goes
-// to pend, which the following product copies over it (kr_row_copy).
+// to pend, which the following product copies over it (gemm_panel_copy_kernel).
 //
 // Same operations in the same order as ln_mix_kernel, kvr_wkv_kernel and
 // gemm_panel_kernel: same bits.
 //
 // Bound: the launch chain (about 4.5 us per launch, 50 launches per step).
-// Measured on MI355X, decode step, us, six launches per layer / four: fp16
-// B = 1 339 / 292, 8 355 / 329, 16 350 / 345, 40 369 / 340, 80 395 / 363,
-// 128 430 / 394, 160 465 / 453, 200 548 / 661; w8a8 B = 1 363 / 301,
-// 16 375 / 374, 40 393 / 377, 128 450 / 418, 144 447 / 466.
+// Measured on MI355X, decode step, us, C = 768, six launches per layer / four:
+// fp16 B = 1 333 / 280, 8 360 / 321, 16 350 / 338, 40 370 / 331, 80 398 / 354,
+// 128 432 / 395, 160 439 / 448, 200 477 / 565; w8a8 B = 1 359 / 292,
+// 16 374 / 363, 40 392 / 366, 128 450 / 404, 144 448 / 454, 200 498 / 596.
 #include <hip/hip_ext.h>
 
 #include <algorithm>
 #include <type_traits>
 
 #include "kr_gemm_epilogue.h"
+#include "kr_panel.h"
 #include "kr_rowops.h"
 #include "kr_step.h"
 #include "kr_wkv.h"
@@ -345,6 +346,51 @@ int launch_rk(const kr_step_rk& a, hipStream_t s) {
     return launch_rk_shape<S, 4, 2, I8>(a, blocks / 2, s);
 }
 
+// The panel product of one job, one row block per workgroup, and a row copy.
+// Bound by the launch chain and the L2 requests in flight, as all panel
+// products. One job only: to select one of kr_gemm_multi's three costs scalar
+// loads that wait for each other (measured on MI355X, one step of 12 layers, us,
+// C = 768, gemm_panel_kernel with the copy in it / this: 1 stream 218 / 212, 128
+// streams 322 / 313; w8a8, 128, 362 / 352).
+struct kr_gemm_one {
+    kr_gemm_args job[1];
+    int ep[1];
+    int tiles[1];
+    unsigned long long* stamps;
+};
+
+template <int NS, int MAXT, bool Q8>
+__global__ void __launch_bounds__(MAXT) gemm_panel_copy_kernel(kr_gemm_one mj, kr_row_copy copy) {
+    panel_product<1, NS, true, Q8, Q8, true>(mj, copy);
+}
+
+template <int NS, int MAXT, bool Q8>
+int launch_product(const kr_gemm_args& g, int ep, const kr_row_copy& copy, hipStream_t s) {
+    const int S = g.K / kKS, blocks = (g.M + 15) / 16 * ((g.N + 16 * NS - 1) / (16 * NS));
+    size_t lds = S > 1 ? (size_t)S * NS * 256 * sizeof(float) : 0;
+    if (Q8 && S > 1) lds += (size_t)S * 16 * sizeof(float);
+    const kr_panel_timing tm = kr_gemm_take_timing(blocks, S);
+    const kr_gemm_one mj{{g}, {ep}, {blocks}, tm.stamps};
+    if (tm.start)
+        hipExtLaunchKernelGGL((gemm_panel_copy_kernel<NS, MAXT, Q8>), dim3(blocks), dim3(64 * S),
+                              (uint32_t)lds, s, tm.start, tm.stop, 0u, mj, copy);
+    else
+        gemm_panel_copy_kernel<NS, MAXT, Q8><<<blocks, 64 * S, lds, s>>>(mj, copy);
+    KR_LAUNCHED();
+    return KR_OK;
+}
+
+template <bool Q8>
+int launch_product(const kr_gemm_args& g, int ep, const kr_row_copy& copy, hipStream_t s) {
+    // one column panel per workgroup while that fits one round of the 256 CUs,
+    // as kr_gemm.hip's busiest-CU model has it at one row block
+    const int S = g.K / kKS;
+    const bool one = (g.M + 15) / 16 * ((g.N + 15) / 16) <= 256;
+    if (S <= 4) return one ? launch_product<1, 256, Q8>(g, ep, copy, s) : launch_product<2, 256, Q8>(g, ep, copy, s);
+    if (S <= 12) return one ? launch_product<1, 768, Q8>(g, ep, copy, s) : launch_product<2, 768, Q8>(g, ep, copy, s);
+    return one ? launch_product<1, 1024, Q8>(g, ep, copy, s) : launch_product<2, 1024, Q8>(g, ep, copy, s);
+}
+
 }  // namespace
 
 int kr_step_launch_kvr(int C, bool i8, const kr_step_kvr& a, hipStream_t s) {
@@ -365,4 +411,13 @@ int kr_step_launch_rk(int C, bool i8, const kr_step_rk& a, hipStream_t s) {
         case 4: return i8 ? launch_rk<4, true>(a, s) : launch_rk<4, false>(a, s);
         default: return kr_fail(KR_EUNSUPPORTED, "C=%d unsupported (256..1024, step 256)", C);
     }
+}
+
+int kr_step_launch_product(const kr_gemm_args& g, int epilogue, const kr_row_copy& copy, hipStream_t s) {
+    const int rc = kr_gemm_check(g, epilogue);
+    if (rc) return rc;
+    KR_REQUIRE(g.a_frag && !g.i8 == !g.a_q16, "step: the product needs fp16 fragment-packed rows");
+    KR_REQUIRE(g.M >= 1 && g.M <= KR_GEMM_SMALL_M && g.N < KR_GEMM_SMALL_MAX_N && g.K / kKS <= 16,
+               "step: product of M=%d N=%d K=%d", g.M, g.N, g.K);
+    return g.i8 ? launch_product<true>(g, epilogue, copy, s) : launch_product<false>(g, epilogue, copy, s);
 }

@@ -108,10 +108,11 @@ def test_step_timing_leaves_the_launches_as_they_are(B, w8a8):
 
 
 # the last row counts of four launches per layer and the first of six, at the
-# widths and codecs whose lines are not among the sizes above
+# widths and codecs whose lines are not among the sizes above; at C = 512, 129
+# rows are also the first with two column panels in the O and V products
 @pytest.mark.parametrize("C,w8a8,Bs", [(256, False, (160, 161)), (256, True, (12, 13, 96, 97, 128, 129)),
-                                       (512, True, (128, 129)), (1024, False, (48, 49)),
-                                       (1024, True, (96, 97))])
+                                       (512, False, (128, 129, 160, 161)), (512, True, (128, 129)),
+                                       (1024, False, (48, 49)), (1024, True, (96, 97))])
 def test_stepped_equals_packed_at_the_lines(C, w8a8, Bs):
     test_stepped_equals_packed(C, Bs, w8a8)
 
