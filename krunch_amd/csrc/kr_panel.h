@@ -60,9 +60,12 @@ typedef unsigned short kr_u16x2 __attribute__((ext_vector_type(2)));
 // only): a row copy rides along (copy is not read otherwise). Its code costs a
 // panel launch four registers and ~0.1 us (and the 2 x 2 tile a wave per SIMD:
 // the channel-mix R/K product at 176 rows 7.0 -> 8.2 us on MI355X), so the
-// launches with one are kernels of their own (kr_step.hip).
+// launches with one are kernels of their own (kr_step.hip). mj is taken by
+// value: by reference the kernel arguments are loaded and selected in another
+// order (12 layers of 7 rows, C = 768, MI355X: 363 against 355 us; w8a8,
+// C = 512, 192 rows 389 / 384).
 template <int TM, int NS, bool FRAG, bool I8, bool QA, bool COPY, class Jobs>
-__device__ __forceinline__ void panel_product(const Jobs& mj, const kr_row_copy& copy) {
+__device__ __forceinline__ void panel_product(Jobs mj, kr_row_copy copy) {
     static_assert(!QA || (I8 && FRAG), "on-load quantisation needs the int8 fragment path");
     constexpr int TT = TM * NS;
     // 1 KB operand blocks per wave slice: 8 x (16x32 fp16) or 4 x (16x64 int8);
