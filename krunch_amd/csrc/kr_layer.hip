@@ -147,6 +147,69 @@ ln_mix_kernel(LnMixArgs a) {
     }
 }
 
+// Packed WKV, one lane per (stream, channel), sequential over T. About 50 VALU
+// instructions per token in one chain per wave, so a window costs ~155 us per
+// 1000 tokens however few streams there are (those go to kr_wkv.hip); with
+// enough waves it is bound by HBM (B = 256: 2.4 GB in 0.51 ms).
+// It stands in this file because, with it in kr_wkv.hip, the LN-mix and K/V/R
+// kernels lie elsewhere in their code object and, instruction for instruction
+// the same, take longer: a step of 12 layers, C = 768, fp16, 192 streams 409
+// against 398 us on MI355X, 161 402 / 392, 320 490 / 478.
+constexpr int kWkvChunk = 16;
+
+template <bool DET>
+__global__ void __launch_bounds__(256) wkv_kernel(const float* __restrict__ k,
+                                                  const float* __restrict__ v,
+                                                  const kr_half* __restrict__ r,
+                                                  const float* __restrict__ decay,
+                                                  const float* __restrict__ first,
+                                                  float* __restrict__ aa, float* __restrict__ bb,
+                                                  float* __restrict__ pp, kr_half* __restrict__ ry,
+                                                  int B, int T, int C, int ry_frag) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    const int b = blockIdx.y;
+    if (c >= C || b >= B) return;
+    const size_t s = (size_t)b * C + c;
+    const size_t base = (size_t)b * T * C + c;
+    const float w = decay[c], u = first[c];
+    WkvState st{aa[s], bb[s], pp[s]};
+    auto ry_at = [&](int t) -> size_t {
+        return ry_frag ? kr_frag_index((long long)b * T + t, c, C) : base + (size_t)t * C;
+    };
+    // A chunk's loads are unconditional (tokens past T re-read token T-1) and
+    // r stays fp16 until its token is computed, so all 3 x kWkvChunk loads are
+    // in flight at once. A load under `t < T` with its conversion beside it
+    // makes the compiler wait for each token's loads in turn (one memory
+    // latency per token).
+    for (int t0 = 0; t0 < T; t0 += kWkvChunk) {
+        float kk[kWkvChunk], vv[kWkvChunk];
+        kr_half rh[kWkvChunk];
+        #pragma unroll
+        for (int q = 0; q < kWkvChunk; q++) {
+            const size_t i = base + (size_t)min(t0 + q, T - 1) * C;
+            kk[q] = k[i];
+            vv[q] = v[i];
+            rh[q] = r[i];
+        }
+        #pragma unroll
+        for (int q = 0; q < kWkvChunk; q++)
+            if (t0 + q < T) ry[ry_at(t0 + q)] = wkv_token<DET>(st, w, u, kk[q], vv[q], (float)rh[q]);
+    }
+    aa[s] = st.a;
+    bb[s] = st.b;
+    pp[s] = st.p;
+}
+
+template <bool DET>
+int wkv_launch(const kr_wkv_args& a, hipStream_t s) {
+    KR_REQUIRE(a.B >= 1 && a.T >= 1 && a.C >= 1, "wkv: bad shape B=%d T=%d C=%d", a.B, a.T, a.C);
+    if (kr_wkv_use_scan(a, DET)) return kr_wkv_launch_scan(a, DET, s);
+    wkv_kernel<DET><<<dim3((a.C + 255) / 256, a.B), 256, 0, s>>>(a.k, a.v, a.r, a.decay, a.first, a.aa, a.bb,
+                                                                 a.pp, a.ry, a.B, a.T, a.C, a.ry_frag);
+    KR_LAUNCHED();
+    return KR_OK;
+}
+
 // ---------------------------------------------------------------------------
 // Stepped K, V, R products fused with the WKV update (T = 1 rows): the three
 // small-M products and wkv_kernel in one launch, with the arithmetic of the
@@ -845,7 +908,7 @@ int layer_forward_q8(const kr_layer_weights& L, int C, int F, kr_half* x, int B,
             KR_TRY(kr_gemm_launch_multi(jobs, eps, 3, s));
         }
         KR_TRY(ph.mark(2));
-        KR_TRY(kr_wkv_launch(wkv_args(L, st, w, B, T, C, fr), true, s));
+        KR_TRY(wkv_launch<true>(wkv_args(L, st, w, B, T, C, fr), s));
     }
     KR_TRY(ph.mark(3));
     if (fr) {
@@ -1004,7 +1067,7 @@ int layer_forward(const kr_layer_weights& L, int C, int F, kr_half* x, int B, in
         KR_TRY(kr_gemm_launch_multi(jobs, eps, 3, s));
     }
     KR_TRY(ph.mark(2));
-    KR_TRY(kr_wkv_launch(wkv_args(L, st, w, B, T, C, fr), false, s));
+    KR_TRY(wkv_launch<false>(wkv_args(L, st, w, B, T, C, fr), s));
     KR_TRY(ph.mark(3));
     KR_TRY(kr_gemm_launch(gemm_args(w.ry, M, C, L.Ot, C, x, x, nullptr, L.Of, fr), KR_EP_RESID, s));
     KR_TRY(ph.mark(4));
@@ -1157,6 +1220,10 @@ int scratch_on_current_device(void** out) {
 }
 
 }  // namespace
+
+int kr_wkv_launch(const kr_wkv_args& a, bool det, hipStream_t s) {
+    return det ? wkv_launch<true>(a, s) : wkv_launch<false>(a, s);
+}
 
 // Entry points used by kr_engine.cpp.
 // ids (nullable): x starts as the embedding of these [B, T] token ids, gathered

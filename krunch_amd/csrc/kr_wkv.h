@@ -1,6 +1,6 @@
 // The WKV recurrence (wkv_kernel.cu:52-73 semantics): one token's update,
-// shared by the packed kernels (kr_wkv.hip) and the stepped K, V, R + WKV
-// kernel (kr_layer.hip), and the packed launch.
+// shared by the packed kernels (wkv_kernel in kr_layer.hip, kr_wkv.hip) and the
+// stepped K, V, R + WKV kernel (kr_layer.hip), and the packed launch.
 #pragma once
 #include "kr_common.h"
 #include "kr_math.h"
@@ -64,3 +64,6 @@ struct kr_wkv_args {
 
 // det: kr_kexp and an IEEE division (the w8a8 codec).
 int kr_wkv_launch(const kr_wkv_args& a, bool det, hipStream_t s);
+// Whether the window goes to the kernel split over time, and its launch (kr_wkv.hip).
+bool kr_wkv_use_scan(const kr_wkv_args& a, bool det);
+int kr_wkv_launch_scan(const kr_wkv_args& a, bool det, hipStream_t s);

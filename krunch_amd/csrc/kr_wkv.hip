@@ -1,14 +1,10 @@
-// Packed WKV (T tokens per stream) and its C-ABI entry point. Two kernels with
-// the operations and bits of wkv_token (kr_wkv.h):
-//
-//  * wkv_kernel: one lane per (stream, channel), sequential over T. About 50
-//    VALU instructions per token in one chain per wave, so a window costs
-//    ~155 us per 1000 tokens however few streams there are; with enough waves
-//    it is bound by HBM (B = 256: 2.4 GB in 0.51 ms).
-//  * wkv_scan_kernel: the serial part of the recurrence is only
-//    p' = max(w + p, k) and a' = f1 a + f2 v, b' = f1 b + f2 (two dependent
-//    operations per token each); the exponentials and the quotient of a token
-//    need nothing but its own p, a, b. A workgroup splits those over waves.
+// Packed WKV (T tokens per stream) split over time, and the C-ABI entry point.
+// wkv_kernel (kr_layer.hip) takes one lane per (stream, channel) and is
+// sequential over T. The serial part of the recurrence is only
+// p' = max(w + p, k) and a' = f1 a + f2 v, b' = f1 b + f2 (two dependent
+// operations per token each); the exponentials and the quotient of a token
+// need nothing but its own p, a, b. A workgroup here splits those over waves.
+// Same operations and bits as wkv_token (kr_wkv.h).
 #include <algorithm>
 
 #include "kr_gemm.h"
@@ -16,51 +12,6 @@
 #include "krunch_hip.h"
 
 namespace {
-
-constexpr int kWkvChunk = 16;
-
-template <bool DET>
-__global__ void __launch_bounds__(256) wkv_kernel(const float* __restrict__ k,
-                                                  const float* __restrict__ v,
-                                                  const kr_half* __restrict__ r,
-                                                  const float* __restrict__ decay,
-                                                  const float* __restrict__ first,
-                                                  float* __restrict__ aa, float* __restrict__ bb,
-                                                  float* __restrict__ pp, kr_half* __restrict__ ry,
-                                                  int B, int T, int C, int ry_frag) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    const int b = blockIdx.y;
-    if (c >= C || b >= B) return;
-    const size_t s = (size_t)b * C + c;
-    const size_t base = (size_t)b * T * C + c;
-    const float w = decay[c], u = first[c];
-    WkvState st{aa[s], bb[s], pp[s]};
-    auto ry_at = [&](int t) -> size_t {
-        return ry_frag ? kr_frag_index((long long)b * T + t, c, C) : base + (size_t)t * C;
-    };
-    // A chunk's loads are unconditional (tokens past T re-read token T-1) and
-    // r stays fp16 until its token is computed, so all 3 x kWkvChunk loads are
-    // in flight at once. A load under `t < T` with its conversion beside it
-    // makes the compiler wait for each token's loads in turn (one memory
-    // latency per token).
-    for (int t0 = 0; t0 < T; t0 += kWkvChunk) {
-        float kk[kWkvChunk], vv[kWkvChunk];
-        kr_half rh[kWkvChunk];
-        #pragma unroll
-        for (int q = 0; q < kWkvChunk; q++) {
-            const size_t i = base + (size_t)min(t0 + q, T - 1) * C;
-            kk[q] = k[i];
-            vv[q] = v[i];
-            rh[q] = r[i];
-        }
-        #pragma unroll
-        for (int q = 0; q < kWkvChunk; q++)
-            if (t0 + q < T) ry[ry_at(t0 + q)] = wkv_token<DET>(st, w, u, kk[q], vv[q], (float)rh[q]);
-    }
-    aa[s] = st.a;
-    bb[s] = st.b;
-    pp[s] = st.p;
-}
 
 // ---------------------------------------------------------------------------
 // 16 channels of one stream per workgroup, the window in chunks of kScanTok
@@ -275,8 +226,7 @@ __global__ void __launch_bounds__(kScanThreads) wkv_scan_kernel(kr_wkv_args g) {
 
 }  // namespace
 
-int kr_wkv_launch(const kr_wkv_args& a, bool det, hipStream_t s) {
-    KR_REQUIRE(a.B >= 1 && a.T >= 1 && a.C >= 1, "wkv: bad shape B=%d T=%d C=%d", a.B, a.T, a.C);
+bool kr_wkv_use_scan(const kr_wkv_args& a, bool det) {
     // The scan kernel up to the stream count where its extra VALU work costs
     // more than wkv_kernel's serial chain. Measured on MI355X at C = 768,
     // T = 1024 (wkv_kernel / scan, us): fp16 B = 20 177 / 79, B = 64 200 / 312
@@ -290,20 +240,13 @@ int kr_wkv_launch(const kr_wkv_args& a, bool det, hipStream_t s) {
     // layer at B = 44 3 us ahead, at B = 53 3 us behind.
     const long long wgs = (long long)a.B * ((a.C + kScanCh - 1) / kScanCh);
     const long long most = a.T < 64 ? (det ? 2048 : 1024) : (det ? 2560 : 1536);
-    const bool scan = a.T >= 32 && wgs <= most;
-    if (scan) {
-        const dim3 grid((a.C + kScanCh - 1) / kScanCh, a.B);
-        if (det) wkv_scan_kernel<true><<<grid, kScanThreads, 0, s>>>(a);
-        else wkv_scan_kernel<false><<<grid, kScanThreads, 0, s>>>(a);
-    } else {
-        const dim3 grid((a.C + 255) / 256, a.B);
-        if (det)
-            wkv_kernel<true><<<grid, 256, 0, s>>>(a.k, a.v, a.r, a.decay, a.first, a.aa, a.bb, a.pp,
-                                                  a.ry, a.B, a.T, a.C, a.ry_frag);
-        else
-            wkv_kernel<false><<<grid, 256, 0, s>>>(a.k, a.v, a.r, a.decay, a.first, a.aa, a.bb,
-                                                   a.pp, a.ry, a.B, a.T, a.C, a.ry_frag);
-    }
+    return a.T >= 32 && wgs <= most;
+}
+
+int kr_wkv_launch_scan(const kr_wkv_args& a, bool det, hipStream_t s) {
+    const dim3 grid((a.C + kScanCh - 1) / kScanCh, a.B);
+    if (det) wkv_scan_kernel<true><<<grid, kScanThreads, 0, s>>>(a);
+    else wkv_scan_kernel<false><<<grid, kScanThreads, 0, s>>>(a);
     KR_LAUNCHED();
     return KR_OK;
 }
