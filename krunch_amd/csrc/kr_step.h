@@ -5,18 +5,16 @@
 // Whether a stepped layer of M streams takes them: beyond, the LN that every
 // column group repeats (C / 16 groups of C values per row) costs more than the
 // launches it saves. Measured on MI355X, one step of 12 layers, F = 4 C, us,
-// six launches per layer / four. fp16: C = 256, M = 16 211 / 191, 160 279 / 214;
-// 512, 16 270 / 224, 160 345 / 268; 768, 16 297 / 265, 128 377 / 316, 144
-// 386 / 368, 160 384 / 376; 1024, 8 343 / 311, 48 357 / 341, 64 386 / 380, 96
-// 403 / 435, 128 429 / 524. w8a8, whose rows are quantised as well: C = 256, 12
-// 239 / 224, 16 243 / 254, 96 267 / 263, 97 297 / 263 (the panel products'
-// tiles change there), 128 305 / 270; 512, 16 306 / 280, 128 357 / 301; 768, 16
-// 327 / 317, 128 401 / 354; 1024, 16 364 / 343, 96 428 / 382, 112 443 / 443.
-// In a decode run of 144 streams (C = 768), whose logits and symbols come
-// between the steps, four are 2 % ahead in fp16 and 1 % behind in w8a8; of 160,
-// 2 % behind in both. Within 2 % the order differs between builds, so no line
-// goes by that. The limits at C <= 512 (fp16) and 512 (w8a8) are the last rows
-// measured ahead, not crossovers.
+// six launches per layer / four. fp16: C = 256, M = 16 213 / 190, 160 275 / 215;
+// 512, 16 267 / 227, 160 346 / 267; 768, 16 291 / 264, 128 369 / 323, 144
+// 371 / 373, 160 372 / 378; 1024, 8 330 / 311, 48 352 / 344, 64 382 / 382, 96
+// 408 / 437, 128 436 / 531. w8a8, whose rows are quantised as well: C = 256, 12
+// 237 / 225, 16 240 / 254, 96 263 / 264, 97 290 / 264 (the panel products'
+// tiles change there), 128 301 / 268; 512, 16 302 / 282, 128 354 / 304; 768, 16
+// 327 / 320, 128 399 / 353; 1024, 16 361 / 346, 96 422 / 382, 112 436 / 445.
+// Decode runs (C = 768): fp16 128 streams 422 / 393, 144 434 / 438; w8a8 128
+// 442 / 405, 144 440 / 455. The limits at C <= 512 (fp16) and 512 (w8a8) are the
+// last rows measured ahead, not crossovers.
 inline bool kr_step_fuse_ok(int C, int M, bool i8) {
     if (i8) return C <= 256 ? M <= 12 || (M > 96 && M <= 128) : M <= (C <= 768 ? 128 : 96);
     return M <= (C <= 512 ? 160 : (C <= 768 ? 128 : 48));

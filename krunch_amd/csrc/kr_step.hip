@@ -19,9 +19,9 @@
 //
 // Bound: the launch chain (about 4.5 us per launch, 50 launches per step).
 // Measured on MI355X, decode step, us, C = 768, six launches per layer / four:
-// fp16 B = 1 333 / 280, 8 360 / 321, 16 350 / 338, 40 370 / 331, 80 398 / 354,
-// 128 432 / 395, 160 439 / 448, 200 477 / 565; w8a8 B = 1 359 / 292,
-// 16 374 / 363, 40 392 / 366, 128 450 / 404, 144 448 / 454, 200 498 / 596.
+// fp16 B = 1 325 / 276, 8 352 / 315, 16 342 / 332, 40 360 / 328, 80 387 / 353,
+// 128 422 / 393, 160 438 / 451, 200 475 / 568; w8a8 B = 1 359 / 290,
+// 16 368 / 361, 40 387 / 364, 128 442 / 405, 144 440 / 455, 200 495 / 595.
 #include <hip/hip_ext.h>
 
 #include <algorithm>
